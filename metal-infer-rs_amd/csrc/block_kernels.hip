@@ -123,6 +123,42 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(RmsNormParams p) {
   }
 }
 
+// The same for narrow rows (width 8 LPR, LPR lanes of one 16-byte piece each: the
+// per-head norms, width 64 to 256), 64 / LPR rows per wave and step, U steps
+// per wave with every load issued before the first sum. A wave per row left most
+// of its lanes idle and its launch bound by the rows' latency.
+template <int LPR, int U>
+__global__ __launch_bounds__(256) void rms_norm_rows_kernel(RmsNormParams p) {
+  constexpr uint32_t RPW = 64 / LPR, ROWS = 4 * RPW * U;  // rows per wave step, per workgroup
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane % LPR;
+  const uint32_t row0 = blockIdx.x * ROWS + wave * (RPW * U) + lane / LPR;
+  const uint4 w = load16(p.weight + 8 * col);
+  uint4 v[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const uint32_t row = min(row0 + RPW * u, p.rows - 1);  // past the last row: re-read, not stored
+    v[u] = load16(p.x + row_offset(p.x_rows, row) + 8 * col);
+  }
+  const uint32_t win[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const float sum = lane_group_sum<LPR>(dot8(v[u], v[u], 0.0f));
+    const float scale = 1.0f / sqrtf(sum / (float)(8 * LPR) + p.epsilon);
+    const uint32_t row = row0 + RPW * u;
+    if (row >= p.rows) continue;
+    const uint32_t vin[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+    uint32_t o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint16_t lo = f32_to_f16(lo_f16(vin[e]) * scale * lo_f16(win[e]));
+      const uint16_t hi = f32_to_f16(hi_f16(vin[e]) * scale * hi_f16(win[e]));
+      o[e] = (uint32_t)lo | ((uint32_t)hi << 16);
+    }
+    *reinterpret_cast<uint4 *>(p.out + row_offset(p.o_rows, row) + 8 * col) =
+        make_uint4(o[0], o[1], o[2], o[3]);
+  }
+}
+
 // rope_f16 (transformer.metal:1514-1531): pairs (i, i + D/2) rotated by
 // (token + offset) * theta^(-2i/D). The same f32 operations, uncontracted,
 // as the fused Q/K kernel's RoPE step.
@@ -455,6 +491,18 @@ hipError_t dispatch_matvec(const MatvecParams &p, bool vec, dim3 grid, const Lau
   return dispatch(matvec_kernel<ROWS, false>, grid, dim3(256), 0, l, p);
 }
 
+// Four steps per wave where that still gives every CU two workgroups, else one
+// (a decode token's heads: the most waves in flight).
+template <int LPR>
+hipError_t launch_rms_rows(const RmsNormParams &p, uint32_t compute_units, const Launch &l) {
+  constexpr uint32_t per_step = 4 * (64 / LPR);
+  if (p.rows >= 4 * per_step * 2 * (uint64_t)compute_units)
+    return dispatch(rms_norm_rows_kernel<LPR, 4>, dim3((p.rows + 4 * per_step - 1) / (4 * per_step)),
+                    dim3(256), 0, l, p);
+  return dispatch(rms_norm_rows_kernel<LPR, 1>, dim3((p.rows + per_step - 1) / per_step), dim3(256), 0,
+                  l, p);
+}
+
 }  // namespace
 
 hipError_t launch_rms_norm(const RmsNormParams &p, uint32_t compute_units, const Launch &l) {
@@ -462,6 +510,12 @@ hipError_t launch_rms_norm(const RmsNormParams &p, uint32_t compute_units, const
   const bool vec = p.width % 8 == 0 && rows_vector_friendly(p.x_rows) &&
                    rows_vector_friendly(p.o_rows) && aligned16(p.x) && aligned16(p.out) &&
                    aligned16(p.weight);
+  if (vec) switch (p.width) {
+      case 64: return launch_rms_rows<8>(p, compute_units, l);
+      case 128: return launch_rms_rows<16>(p, compute_units, l);
+      case 256: return launch_rms_rows<32>(p, compute_units, l);
+      default: break;
+    }
   const dim3 grid((p.rows + 3) / 4);
   // Grids smaller than the CUs load the weights with the row (one round
   // trip less); larger ones keep the later load, which holds more waves.

@@ -307,6 +307,19 @@ def test_rms_norm_parity(ctx, shape):
     check_rms_norm(got, x, w, 1e-6, str(shape))
 
 
+@pytest.mark.parametrize("width", [64, 128, 256])
+@pytest.mark.parametrize("rows", [1, 33, 4 * 32 * 2 * 256 + 5])
+def test_rms_norm_narrow_rows(ctx, width, rows):
+    """Several rows per wave: the last wave part filled, one and four steps per
+    wave, input rows of a strided view."""
+    store = rand(rows + width, (rows, width + 8))
+    w = rand(7, (width,), scale=0.3)
+    dev = ctx.tensor(store)  # views do not keep their storage alive
+    view = dev.view((rows, width), (width + 8, 1))
+    got = ctx.download(ctx.rms_norm(view, ctx.tensor(w), 1e-6))
+    check_rms_norm(got, np.ascontiguousarray(store[:, :width]), w, 1e-6, f"{rows}x{width}")
+
+
 def test_rms_norm_on_a_head_view_of_a_fused_projection(ctx):
     """Query heads as a [T, 16, 128] view of a [T, 32 * 128] buffer."""
     T = 6
