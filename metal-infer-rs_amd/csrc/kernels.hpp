@@ -67,6 +67,7 @@ struct RowsParams {
   uint32_t query_offset;    // ignored when lengths != null
   uint32_t block_keys;      // keys per split
   uint32_t max_splits;
+  uint32_t rows;               // MFMA decode: packed (token, head) rows of a partial (at most 16)
   uint32_t stream_workgroups;  // stream-K decode: workgroups of the launch
   uint32_t stream_unit_slots;  // stream-K decode: fixed partial slots per unit (0 or kStreamUnitSlots)
   float scale_log2;         // rsqrt(D) * log2(e)
@@ -180,6 +181,17 @@ hipError_t launch_rows(const RowsParams &p, uint32_t head_dim, uint32_t waves,
                        uint32_t chunk, RowsPhase phase, const Launch &l);
 // Largest head chunk (of 8, 4, 2, 1) that divides `group`.
 uint32_t rows_chunk(uint32_t group);
+
+// Few-row split-K attention on MFMA (head_dim 64 and 128, 8 waves): at
+// most kDecodeRows packed (token, head) rows per KV head and chunk, heads cut
+// into head_chunks chunks of ceil(group / head_chunks) (one chunk with several
+// tokens). RowsParams as for the rows kernel; `partial` is [units][max_splits],
+// each rows * (D + 2) floats; the last split of a unit merges (counters
+// required). With step_k set (head_dim 128) a decode step, as above. A full
+// 32-key tile of K or V must span less than 4 GiB.
+constexpr uint32_t kDecodeRows = 16;
+constexpr uint32_t kDecodeWaves = 8;
+hipError_t launch_decode(const RowsParams &p, uint32_t head_dim, const Launch &l);
 
 // Batched decode (one query token per sequence, head_dim 128) on MFMA with
 // a stream-K split: p.stream_workgroups workgroups share the keys of all

@@ -16,12 +16,13 @@
 namespace mi {
 namespace {
 
-enum class Family { Naive, Rows, Prefill };
+enum class Family { Naive, Rows, Decode, Prefill };
 
 struct AttnPlan {
   Family family = Family::Rows;
   uint32_t T = 0, Hq = 0, Hkv = 0, D = 0, L = 0, G = 0;
   uint32_t waves = 4, chunk = 1, block_keys = 0, splits = 1;
+  uint32_t head_chunks = 1;      // decode: chunks of a KV head's query heads
   bool fused = false;            // rows: the last split merges (no merge launch)
   uint64_t units = 0;            // rows-kernel (row, KV head, chunk) units
   uint64_t scratch_bytes = 0;
@@ -128,6 +129,60 @@ mi_status plan_rows(const Context *ctx, AttnPlan *p, uint64_t batch, uint32_t ma
   p->grid[1] = p->Hkv * (p->G / p->chunk);
   p->grid[2] = (uint32_t)(batch * p->T);
   return MI_OK;
+}
+
+// Whether the few-row MFMA kernel (attn_decode.hip) is the faster one for T tokens
+// over `keys` keys. The rows kernel spends vector arithmetic on every (row, key),
+// and one workgroup of it on every head chunk and token; the MFMA kernel has the
+// longer fixed chain. Measured on MI355X (graph replays, rotated caches; rows /
+// MFMA us): 8-head chunks 64/8 heads at 300 keys 13.3 / 9.6, 100 keys 10.0 / 5.2;
+// 4-head chunks, one or two tokens, 32/8 at 100 keys 6.4 / 5.2, 1000 keys 9.2 /
+// 9.0, 2 x 500 10.7 / 9.8. Smaller chunks cross at a number of (row, key) pairs
+// that grows with the rows to merge: 16/8 at 4095 keys 9.3 / 9.5, 5000 11.5 /
+// 10.3; 40/8 (five one-head chunks) at 1000 7.8 / 9.4, 2000 10.9 / 9.9; 2 tokens
+// of 16/8 at 1500 8.5 / 9.3, 3000 9.9 / 9.7; 4 of 32/8 at 1500 12.3 / 13.0, 6000
+// 25.4 / 15.7. At head_dim 64 the fixed chain is shorter: 16/8 at 300 to 2000
+// keys 6.6-7.1 / 6.6-7.0, 32/8 at 300 8.9 / 6.7, 40/8 at 400 6.0 / 7.3. The
+// decode step's transforms lengthen the chain, so its 4-head chunks cross later
+// (32/8 at 2000 keys 10.7 / 10.9; 64/8 at 300 15.5 / 11.2).
+bool decode_mfma_wins(const AttnPlan &p, uint64_t keys, bool step) {
+  const uint32_t chunk = kernels::rows_chunk(p.G), rows = p.T * p.G;
+  if (p.T <= 2 && chunk >= (p.D == 64 ? 2u : step ? 8u : 4u)) return true;
+  const uint64_t cross = 6144 + 1280 * (uint64_t)rows;
+  return rows * keys >= (p.D == 64 ? cross / 2 : cross);
+}
+
+// The few-row MFMA kernel's plan: about one 8-wave workgroup per CU, each with at
+// least 128 keys (half its waves busy: 192 or 256 measured slower at every
+// length, 2047 keys 9.3 against 8.7 us). False if it cannot or should not run.
+bool plan_decode(const Context *ctx, AttnPlan *p, uint32_t max_keys, bool step) {
+  if ((p->D != 64 && p->D != 128) || p->T == 0 || p->G == 0 || max_keys == 0) return false;
+  if (p->T > 1 && (uint64_t)p->T * p->G > kernels::kDecodeRows) return false;
+  if (!decode_mfma_wins(*p, max_keys, step)) return false;
+  const uint32_t chunks = p->T == 1 ? ceil_div(p->G, kernels::kDecodeRows) : 1;
+  const uint32_t rows = ceil_div(p->G, chunks) * p->T;
+  const uint64_t units = (uint64_t)p->Hkv * chunks;
+  const uint64_t counters = ctx ? ctx->split_counter_count : kernels::kSplitCounters;
+  if (units > counters || units > 0xffffu) return false;
+  const uint64_t cus = std::max<uint32_t>(ctx ? ctx->compute_units : 256, 1);
+  const uint32_t splits = (uint32_t)std::max<uint64_t>(
+      1, std::min<uint64_t>(ceil_div(max_keys, 128), cus / units));
+  p->family = Family::Decode;
+  p->kernel = "attn_rows";
+  p->waves = kernels::kDecodeWaves;
+  p->threads = p->waves * 64;
+  p->block_keys = ceil_div(ceil_div(max_keys, splits), 32) * 32;
+  p->splits = ceil_div(max_keys, p->block_keys);
+  p->fused = true;
+  p->chunk = rows;
+  p->head_chunks = chunks;
+  p->units = units;
+  p->scratch_bytes =
+      p->splits > 1 ? units * p->splits * rows * (uint64_t)(p->D + 2) * sizeof(float) : 0;
+  p->grid[0] = p->splits;
+  p->grid[1] = (uint32_t)units;
+  p->grid[2] = 1;
+  return true;
 }
 
 // Key tiles of each prefill row tile: the kernel's causal window of the row
@@ -348,6 +403,13 @@ mi_status plan_attention(const Context *ctx, const mi_tensor *q, const mi_tensor
   uint32_t rows_threads = 256;
   if (kind == MI_ATTN_FLASH_DECODE) rows_threads = flash_default ? 0 : flash_threads;
   if (kind == MI_ATTN_DECODE_SPLIT_KV) rows_threads = 0;
+  // Explicit and tuned FlashDecode configurations name the rows kernel's splits.
+  if ((kind != MI_ATTN_FLASH_DECODE || flash_default) &&
+      pos_stride_fits_u32(k->stride[0], v->stride[0], 32) &&
+      plan_decode(ctx, &p, available_last, false)) {
+    *plan = p;
+    return MI_OK;
+  }
   st = plan_rows(ctx, &p, 1, available_last, rows_block, rows_threads);
   if (st != MI_OK) return st;
   *plan = p;
@@ -378,8 +440,17 @@ mi_status run_rows(Batch *batch, const AttnPlan &p, kernels::RowsParams rp,
   rp.counter_stride = kernels::counter_stride(p.units, ctx->split_counter_count);
   rp.block_keys = p.block_keys;
   rp.max_splits = p.splits;
-  rp.head_chunks = p.G / p.chunk;
   rp.group = p.G;
+  if (p.family == Family::Decode) {
+    rp.head_chunks = p.head_chunks;
+    rp.rows = p.chunk;
+    st = launch(batch, p.kernel, [&](const kernels::Launch &s) {
+      return kernels::launch_decode(rp, p.D, s);
+    }, events);
+    scratch_give(ctx, src, scratch);
+    return st;
+  }
+  rp.head_chunks = p.G / p.chunk;
   st = launch(batch, p.kernel, [&](const kernels::Launch &s) {
     return kernels::launch_rows(rp, p.D, p.waves, p.chunk, kernels::RowsPhase::Split, s);
   }, events);
@@ -949,7 +1020,14 @@ mi_status mi_decode_step_attention(mi_batch *batch, const mi_tensor *q, const mi
   if ((st = plan_attention(batch->ctx, q, &key, &val, config, MI_ATTN_DECODE_SPLIT_KV, 0, 0, false,
                            out, &p)) != MI_OK)
     return st;
-  const bool fused = p.family == Family::Rows && p.D == 128 && p.waves == 8 &&
+  // The step's own choice between the two kernels, over the cached keys (the new
+  // one comes from registers in the MFMA kernel).
+  if (p.family != Family::Naive && p.D == 128) {
+    const uint32_t cached = std::max<uint32_t>(1, qk_config->offset);
+    if (!pos_stride_fits_u32(key.stride[0], val.stride[0], 32) || !plan_decode(batch->ctx, &p, cached, true))
+      if ((st = plan_rows(batch->ctx, &p, 1, p.L, 0, 0)) != MI_OK) return st;
+  }
+  const bool fused = p.family != Family::Naive && p.D == 128 && p.waves == 8 &&
                      vector_friendly(*k, 8) && vector_friendly(*value, 8) &&
                      vector_friendly(*key_cache, 8) && vector_friendly(*value_cache, 8) &&
                      reinterpret_cast<uintptr_t>(q_weight->data) % 16 == 0 &&

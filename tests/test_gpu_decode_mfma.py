@@ -1,0 +1,99 @@
+"""The few-row MFMA attention (attn_decode.hip) at the edges of its tiles, splits, head
+chunks and row packing, against the oracle."""
+import numpy as np
+import pytest
+
+import mi_attn
+import oracle
+from helpers import KINDS, assert_parity, f16, oracle_attention, run_attention, upload_kv
+
+pytestmark = pytest.mark.gpu
+
+
+def rand(seed, shape, scale=1.0):
+    return (scale * np.random.default_rng(seed).standard_normal(shape)).astype(np.float16).view(np.uint16)
+
+
+@pytest.mark.parametrize("hq,hkv,d,T,off,extra,causal,kind", [
+    (8, 1, 128, 1, 0, 0, True, "flash-decode"),        # one key
+    (64, 8, 128, 1, 31, 0, True, "decode-split-kv"),   # one whole tile, one split
+    (64, 8, 128, 1, 128, 0, True, "flash-decode"),     # a second split of one key
+    (32, 8, 128, 1, 255, 9, True, "flash-decode"),     # keys past the window are not read
+    (32, 8, 128, 1, 99, 57, False, "flash-decode"),    # non-causal: every key
+    (64, 8, 128, 1, 4999, 0, True, "flash-decode"),    # 32 splits: a whole merge pass
+    (8, 1, 128, 1, 9000, 0, True, "flash-decode"),     # 71 splits: three merge passes
+    (17, 1, 128, 1, 2300, 0, True, "flash-decode"),    # two head chunks of 9 and 8
+    (40, 2, 64, 1, 777, 0, True, "decode-split-kv"),   # two head chunks of 10
+    (32, 8, 64, 1, 300, 0, True, "flash-decode"),
+    (16, 8, 64, 1, 5000, 0, True, "flash-decode"),
+    (32, 8, 128, 2, 30, 0, True, "tiled"),             # two tokens, windows across a tile edge
+    (32, 8, 128, 4, 3001, 0, True, "tiled"),           # 16 rows
+    (15, 3, 128, 3, 4000, 5, True, "tiled"),           # 15 rows of 5 heads
+    (16, 8, 64, 8, 1900, 0, False, "tiled"),
+    (12, 1, 64, 1, 2047, 0, True, "tiled"),
+])
+def test_few_row_attention(ctx, hq, hkv, d, T, off, extra, causal, kind):
+    L = off + T + extra
+    q, k, v = rand(1, (T, hq, d), 2.0), rand(2, (L, hkv, d)), rand(3, (L, hkv, d))
+    geo = dict(hq=hq, hkv=hkv, d=d, off=off, causal=causal)
+    qt, (ko, kview) = ctx.tensor(q), upload_kv(ctx, k, "head_major")
+    info = ctx.plan(qt, kview, kview, mi_attn.AttentionConfig(hq, hkv, d, causal, off), KINDS[kind])
+    group, chunks = hq // hkv, 1 if T > 1 else -(-hq // hkv // 16)
+    rows = T * -(-group // chunks)
+    assert info["block_threads"] == 512 and info["grid"][1] == hkv * chunks, info
+    assert info["scratch_bytes"] in (0, info["grid"][1] * info["splits"] * rows * (d + 2) * 4), info
+    out = run_attention(ctx, q, k, v, kind=kind, layout="position_major", **geo)
+    again = run_attention(ctx, q, k, v, kind=kind, layout="head_major", **geo)
+    # f16 inputs, f32 probabilities (22 bits in the products) and sums: one
+    # rounding of the output, a few f32 roundings of the sums before it.
+    ref = oracle_attention(q, k, v, **geo)["f32"]
+    bound = np.abs(ref) * 2.0 ** -11 + 2.0 ** -24 + 1e-5
+    assert (np.abs(f16(out).astype(np.float64) - ref) <= bound).all()
+    assert (again == out).all()
+
+
+@pytest.mark.parametrize("d,T,off,kind", [(128, 1, 2300, "flash-decode"), (64, 1, 700, "flash-decode"),
+                                          (128, 2, 400, "tiled")])
+def test_few_row_attention_with_infinite_values(ctx, d, T, off, kind):
+    """An infinite value reaches the rows that see its key and no others, as a weighted sum over
+    the visible keys gives it."""
+    hq, hkv, L = 8, 1, off + T
+    q, k, v = rand(4, (T, hq, d)), rand(5, (L, hkv, d)), rand(6, (L, hkv, d))
+    v[L - 1, 0, 5] = np.float16(np.inf).view(np.uint16)      # the last token's own key
+    v[off // 2, 0, d - 1] = np.float16(-np.inf).view(np.uint16)
+    geo = dict(hq=hq, hkv=hkv, d=d, off=off)
+    ref = oracle_attention(q, k, v, **geo)["f32"]
+    got = f16(run_attention(ctx, q, k, v, kind=kind, **geo))
+    assert (np.isposinf(ref) == np.isposinf(got)).all() and (np.isneginf(ref) == np.isneginf(got)).all()
+    fine = np.isfinite(ref)
+    assert np.isfinite(got[fine]).all() and np.abs(got[fine] - ref[fine]).max() <= 2e-3
+
+
+@pytest.mark.parametrize("hq,hkv,pos", [(64, 8, 0), (64, 8, 32), (8, 1, 300), (40, 2, 129), (32, 8, 3500),
+                                        (17, 1, 900)])
+def test_decode_step_on_the_mfma_kernel(ctx, hq, hkv, pos):
+    """The one-launch step: no cached key, splits and head chunks; the cache row that it writes is
+    the only one that changes, and what the row held before has no influence."""
+    d, cap = 128, pos + 2
+    q, k, v = rand(1, (1, hq, d)), rand(2, (1, hkv, d)), rand(3, (1, hkv, d))
+    qw, kw = rand(4, (d,), 0.3), rand(5, (d,), 0.3)
+    hist_k, hist_v = rand(6, (cap, hkv, d)), rand(7, (cap, hkv, d))
+    hist_k[pos], hist_v[pos] = 0x7e00, 0x7e00  # NaN until the step writes it
+    cache = ctx.kv_cache(1, hkv, d, cap)
+    key, value = cache.layer(0)
+    ctx.upload(key, hist_k)
+    ctx.upload(value, hist_v)
+    tensors = [ctx.tensor(x) for x in (q, k, v, qw, kw)]
+    batch = ctx.begin_batch()
+    out = batch.decode_step_attention(*tensors, key, value, mi_attn.QkNormRopeCacheConfig(pos, 1e6, 1e-6),
+                                      mi_attn.AttentionConfig(hq, hkv, d, True, pos))
+    batch.finish()
+    got, key_now, value_now = ctx.download(out), ctx.download(key), ctx.download(value)
+    others = np.arange(cap) != pos
+    assert (key_now[others] == hist_k[others]).all() and (value_now[others] == hist_v[others]).all()
+    assert (value_now[pos] == v[0]).all()
+    want_q, want_k = oracle.qk_norm_rope(q, k, qw, kw, offset=pos, theta=1e6, epsilon=1e-6)
+    assert np.abs(f16(key_now[pos]) - f16(want_k[0])).max() <= 2e-3
+    ref = oracle_attention(want_q, key_now[:pos + 1], value_now[:pos + 1], hq=hq, hkv=hkv, d=d, off=pos)
+    assert_parity(got, ref, label=f"{hq}/{hkv} pos {pos}")
+    cache.close()
