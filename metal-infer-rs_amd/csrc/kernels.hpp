@@ -305,6 +305,19 @@ constexpr uint32_t prefill_workgroups_per_cu(uint32_t head_dim) { return head_di
 // past its row tile's last key tile returns at once. Q, K, V and the output
 // rows are 16-byte aligned (base and outer strides multiples of 8 elements).
 hipError_t launch_prefill(const PrefillParams &p, uint32_t head_dim, const Launch &l);
+
+// Tiled attention of several tokens on MFMA (head_dim 64 and 128), with f32
+// probabilities (two f16 terms) and partials. PrefillParams with block_m 128;
+// grid (splits, row_tiles, kv_heads), split z covering key tiles [z *
+// split_tiles, (z + 1) * split_tiles) or all of them with one split. With more
+// splits `partial` holds tiled_partial_floats floats and the Merge phase (next
+// on the same stream) combines them. Alignment as for launch_prefill.
+enum class TiledPhase { Split, Merge };
+constexpr uint64_t tiled_partial_floats(uint64_t splits, uint64_t row_tiles, uint64_t kv_heads,
+                                        uint64_t head_dim) {
+  return splits * row_tiles * kv_heads * 4 * 64 * (head_dim / 2 + 2);
+}
+hipError_t launch_tiled(const PrefillParams &p, uint32_t head_dim, TiledPhase phase, const Launch &l);
 // Capacity of a context's split-K arrival counters (u32 words: units of a
 // fused rows plan, row tiles x KV heads of a split prefill grid, each at
 // counter_stride words).

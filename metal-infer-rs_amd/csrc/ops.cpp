@@ -16,7 +16,7 @@
 namespace mi {
 namespace {
 
-enum class Family { Naive, Rows, Decode, Prefill };
+enum class Family { Naive, Rows, Decode, Tiled, Prefill };
 
 struct AttnPlan {
   Family family = Family::Rows;
@@ -284,6 +284,40 @@ void order_prefill_pieces(const Context *ctx, AttnPlan *p, bool causal, uint32_t
   p->grid[2] = 1;
 }
 
+// The Tiled kind's MFMA plan for more rows than the few-row kernel takes (or fewer
+// where that one loses): about one workgroup per CU, the keys split into ranges of
+// at least two tiles where the row tiles do not fill the chip (two workgroups per
+// CU measured the same with twice the partials; fewer than 8 key tiles are not
+// split, 200 tokens of 32/8 heads alone 10.8 against 13.2 us). The rows kernel
+// reads every key again for every token; small calls are still faster on it
+// (measured on MI355X, rows / this: 16/8 heads, 10 tokens on 300 keys 8.3 / 10.6
+// us, 32/8, 10 on 500 13.7 / 10.1, 64/8, 4 on 2000 19.9 / 13.0, 32/8, 24 on 6000
+// 108 / 20, 16/8, 2000 alone 473 / 55).
+bool plan_tiled(const Context *ctx, AttnPlan *p, uint32_t max_keys) {
+  if ((p->D != 64 && p->D != 128) || p->T <= 1 || p->G == 0 || max_keys == 0) return false;
+  const uint64_t rows = (uint64_t)p->T * p->G;
+  if (rows >= (1ull << 31) || rows * max_keys < 12000) return false;
+  const uint64_t cus = std::max<uint32_t>(ctx ? ctx->compute_units : 256, 1);
+  const uint32_t row_tiles = ceil_div(rows, kernels::kPrefillBlockM);
+  if (row_tiles > 0xffffu || p->Hkv > 0xffffu) return false;
+  const uint64_t wgs = (uint64_t)row_tiles * p->Hkv;
+  const uint32_t tiles = ceil_div(max_keys, kernels::kPrefillBlockN);
+  const uint32_t want =
+      tiles < 8 ? 1 : (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(tiles / 2, cus / wgs));
+  const uint32_t per_split = ceil_div(tiles, want);
+  p->family = Family::Tiled;
+  p->kernel = "attn_tiled";
+  p->threads = 256;
+  p->splits = ceil_div(tiles, per_split);
+  p->block_keys = p->splits > 1 ? per_split * kernels::kPrefillBlockN : 0;
+  p->grid[0] = p->splits;
+  p->grid[1] = row_tiles;
+  p->grid[2] = p->Hkv;
+  p->scratch_bytes =
+      p->splits > 1 ? kernels::tiled_partial_floats(p->splits, row_tiles, p->Hkv, p->D) * sizeof(float) : 0;
+  return true;
+}
+
 mi_status plan_attention(const Context *ctx, const mi_tensor *q, const mi_tensor *k,
                          const mi_tensor *v, const mi_attention_config *config, int32_t kind,
                          uint32_t block_keys, uint32_t threads, bool flash_explicit,
@@ -410,6 +444,13 @@ mi_status plan_attention(const Context *ctx, const mi_tensor *q, const mi_tensor
     *plan = p;
     return MI_OK;
   }
+  if (kind == MI_ATTN_TILED && vector_friendly(*q, 8) && vector_friendly(*k, 8) &&
+      vector_friendly(*v, 8) && (out == nullptr || vector_friendly(*out, 8)) &&
+      pos_stride_fits_u32(k->stride[0], v->stride[0], kernels::kPrefillBlockN) &&
+      plan_tiled(ctx, &p, available_last)) {
+    *plan = p;
+    return MI_OK;
+  }
   st = plan_rows(ctx, &p, 1, available_last, rows_block, rows_threads);
   if (st != MI_OK) return st;
   *plan = p;
@@ -507,7 +548,7 @@ mi_status run_attention(Batch *batch, const mi_tensor *q, const mi_tensor *k,
     if (scores != nullptr) scratch_free(batch->ctx, scores);
     return st;
   }
-  if (p.family == Family::Prefill) {
+  if (p.family == Family::Prefill || p.family == Family::Tiled) {
     kernels::PrefillParams pp{};
     pp.q = qd, pp.q_tok = q->stride[0], pp.q_head = q->stride[1];
     pp.k = kd, pp.k_pos = k->stride[0], pp.k_head = k->stride[1];
@@ -528,6 +569,17 @@ mi_status run_attention(Batch *batch, const mi_tensor *q, const mi_tensor *k,
       if ((st = scratch_alloc(batch, p.scratch_bytes, &scratch)) != MI_OK) return st;
     }
     pp.partial = static_cast<float *>(scratch);
+    if (p.family == Family::Tiled) {
+      st = launch(batch, p.kernel, [&](const kernels::Launch &s) {
+        return kernels::launch_tiled(pp, p.D, kernels::TiledPhase::Split, s);
+      });
+      if (st == MI_OK && p.splits > 1)
+        st = launch(batch, "attn_tiled_merge", [&](const kernels::Launch &s) {
+          return kernels::launch_tiled(pp, p.D, kernels::TiledPhase::Merge, s);
+        });
+      if (scratch != nullptr) scratch_free(batch->ctx, scratch);
+      return st;
+    }
     pp.counters = batch->ctx->split_counters;
     pp.counter_stride =
         kernels::counter_stride((uint64_t)pp.row_tiles * p.Hkv, batch->ctx->split_counter_count);
