@@ -281,9 +281,10 @@ mi_status mi_attention_plan(const mi_context *ctx, const mi_tensor *q,
  * (values above C are clamped to C; a sequence of length 0 gets NaN, the
  * reference's 0/0); causal over each sequence (query at position
  * lengths[b] - 1). out [B, Hq, D]. config->query_offset is ignored.
- * block_keys = 0 picks the default: at head_dim 128 and B <= 1024 an MFMA
- * kernel whose workgroups share all sequences' keys equally (stream-K),
- * otherwise the rows kernel over a flat (sequence, KV head, split) grid.
+ * block_keys = 0 picks the default: at head_dim 128, and mostly at 64, with
+ * B <= 1024 an MFMA kernel whose workgroups share all sequences' keys equally
+ * (stream-K; few keys: one piece of a unit per workgroup), otherwise the rows
+ * kernel over a flat (sequence, KV head, split) grid.
  * block_keys > 0 runs the rows kernel with splits of that many keys. */
 mi_status mi_attention_decode_batched(mi_batch *batch, const mi_tensor *q,
                                       const mi_tensor *k, const mi_tensor *v,

@@ -618,7 +618,9 @@ __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(
 
 // ---------------------------------------------------------------------------
 // Batched decode on MFMA with a stream-K split (one query token per sequence,
-// D = 128). Measured on MI355X at 32 sequences, L ~ U[1024, 8192], GQA 4:
+// D = 64 and 128; a unit's heads are any group, up to 16 of them: 40/8 heads read
+// K/V once instead of once per power-of-two chunk, 71 sequences of 630 to 811
+// keys 176.6 -> 49.6 us). Measured on MI355X at 32 sequences, L ~ U[1024, 8192], GQA 4:
 // 110 us against 126 us for the rows kernel with 768-key splits.
 //  - Work split: the launch's workgroups divide the flattened (unit, key)
 //    space of all sequences (unit = sequence, KV head, head chunk) into equal
@@ -663,23 +665,43 @@ __device__ __forceinline__ int stream_slot_key(int r) {
   return (((r >> 2) & 1) << 4) | (((r >> 3) & 3) << 2) | (r & 3);
 }
 // XOR applied to the 32-byte column pair of V row r: the 16 rows of one
-// transposed read then fall on 8 distinct bank groups.
-__device__ __forceinline__ int stream_swizzle(int r) { return (r & 3) | (((r >> 3) & 1) << 2); }
+// transposed read then fall on 8 distinct bank groups (D = 64: rows are half a
+// bank row, so their parity already picks one of two halves).
+template <int D>
+__device__ __forceinline__ int stream_swizzle(int r) {
+  return D == 128 ? ((r & 3) | (((r >> 3) & 1) << 2)) : (((r >> 1) & 1) | (((r >> 3) & 1) << 1));
+}
 
-template <int GC>
-__global__ __launch_bounds__(kStreamWaves * 64, 2) void attn_decode_stream_kernel(
+// Workgroups per CU of the stream kernel's launch (three at D = 64 measured
+// slower: 32 sequences of 1024 to 8192 keys 64.7 against 60.6 us).
+constexpr int kStreamPerCu = 2;
+
+// D = 64 keeps the precision of the rows kernel that served it: probabilities
+// are f32 values carried into P V as two f16 terms (hi + lo, 22 bits; twice the
+// P V MFMAs, which its bound, HBM, hides). Measured on MI355X, rows kernel ->
+// this with its merge launch: 70 sequences of 100 to 4000 keys, 32/8 heads 75.9
+// -> 71.1 us; 32 of 1024 to 8192 71.4 -> 60.6; 128 of 100 to 1500 66.8 -> 57.2;
+// 14 of 745 to 1456, 64/8 heads 31.6 -> 18.2.
+template <int D>
+__global__ __launch_bounds__(kStreamWaves * 64, kStreamPerCu) void attn_decode_stream_kernel(
     const RowsParams p) {
-  constexpr int D = 128, WAVES = kStreamWaves, KT = kStreamTile, DC = D / 32, DB = D / 16;
+  constexpr int WAVES = kStreamWaves, KT = kStreamTile, DC = D / 32, DB = D / 16;
+  constexpr int CPR = D / 8, VL = KT * CPR / 64;  // 16-byte chunks per V row, 1 KB V loads per tile
+  constexpr bool SPLIT_P = D == 64;
+  // Added to every weight's exponent, so that low terms stay above f16's
+  // smallest values; it cancels between the weighted sum and the row sum.
+  constexpr float kBias = SPLIT_P ? 6.0f : 0.0f;
   constexpr int THREADS = WAVES * 64;
   constexpr int STAGE = KT * D;  // halves of V per wave and stage
-  static_assert(WAVES * GC * D * 4 <= WAVES * STAGE * 2, "wave merge must fit a stage");
+  constexpr int GM = kDecodeRows;  // most heads of a chunk
+  static_assert(WAVES * GM * D * 4 <= WAVES * STAGE * 2, "wave merge must fit a stage");
   // Two V stages, one array each, so the compiler can tell the direct loads
   // into one from the reads of the other. After a piece's tile loop stage a
   // holds the wave merge.
   __shared__ __attribute__((aligned(16))) uint16_t v_lds_a[WAVES * STAGE];
   __shared__ __attribute__((aligned(16))) uint16_t v_lds_b[WAVES * STAGE];
-  __shared__ float s_m[WAVES][GC];
-  __shared__ float s_l[WAVES][GC];
+  __shared__ float s_m[WAVES][GM];
+  __shared__ float s_l[WAVES][GM];
   __shared__ uint64_t s_pre[kStreamMaxBatch + 1];  // keys of all units before sequence b
   __shared__ uint32_t s_len[kStreamMaxBatch];      // visible keys of sequence b
 
@@ -720,6 +742,48 @@ __global__ __launch_bounds__(kStreamWaves * 64, 2) void attn_decode_stream_kerne
     if (lane == 0) s_pre[0] = 0;
   }
   __syncthreads();
+  // Few keys: pieces of one unit each, of the smallest size that gives every
+  // piece its own workgroup, instead of equal segments, whose boundaries would
+  // leave most workgroups two short pieces (each a full latency chain) in turn.
+  // s_pre then counts pieces. Measured on MI355X, equal segments of at least 512
+  // keys -> this (and of at least 128 keys past it): 8 sequences of 40 to 1000
+  // keys, 16/8 heads 21.7 -> 13.2 us; 16 of 100 to 900, 32/8 28.1 -> 18.8; 4 of
+  // 3000 to 5000 30.8 -> 26.0; 128 of 10 to 100 77.9 -> 42.6; 512-key pieces lost
+  // where they run (20 of 500 to 1500: 28.7 against 25.7 in segments).
+  uint32_t piece_keys = 0;
+  if (s_pre[p.batch] <= (uint64_t)gridDim.x * kStreamPieceMost) {
+    uint32_t count[2] = {0, 0};  // pieces of kStreamMinKeys and of kStreamPieceMost keys
+    for (uint32_t c0 = 0; c0 < p.batch; c0 += 64) {
+      const uint32_t n = c0 + lane < p.batch ? s_len[c0 + lane] : 0;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const uint32_t size = i == 0 ? kStreamMinKeys : kStreamPieceMost;
+        uint32_t c = (n + size - 1) / size;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) c += __shfl_xor(c, d, 64);
+        count[i] += c;
+      }
+    }
+    if ((uint64_t)count[1] * upb <= gridDim.x) piece_keys = kStreamPieceMost;
+    if ((uint64_t)count[0] * upb <= gridDim.x) piece_keys = kStreamMinKeys;
+  }
+  if (piece_keys != 0) {
+    __syncthreads();
+    if (wave == 0) {
+      uint32_t carry = 0;
+      for (uint32_t c0 = 0; c0 < p.batch; c0 += 64) {
+        uint32_t x = c0 + lane < p.batch ? (s_len[c0 + lane] + piece_keys - 1) / piece_keys * upb : 0;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+          const uint32_t y = __shfl_up(x, d, 64);
+          if (lane >= d) x += y;
+        }
+        if (c0 + lane < p.batch) s_pre[c0 + lane + 1] = carry + x;
+        carry += __shfl(x, 63, 64);
+      }
+    }
+    __syncthreads();
+  }
   // Sequences with no key: the reference divides 0 by 0.
   for (uint32_t b = blockIdx.x; b < p.batch; b += gridDim.x)
     if (s_pre[b + 1] == s_pre[b])
@@ -727,7 +791,8 @@ __global__ __launch_bounds__(kStreamWaves * 64, 2) void attn_decode_stream_kerne
         p.out[(int64_t)b * p.o_seq + (int64_t)(idx / D) * p.o_head + idx % D] = 0x7e00;
   const uint64_t total = s_pre[p.batch];
   // At least kStreamMinKeys per workgroup; the rest of the grid idles.
-  const uint64_t W = min((uint64_t)gridDim.x, max((uint64_t)1, total / kStreamMinKeys));
+  // (Pieces: one position per workgroup.)
+  const uint64_t W = piece_keys != 0 ? max((uint64_t)1, total) : min((uint64_t)gridDim.x, max((uint64_t)1, total / kStreamMinKeys));
   // 32-bit division when the total fits (a 64-bit one is a long sequence).
   const uint64_t seg = total + W - 1 <= 0xffffffffull
                            ? (uint64_t)((uint32_t)(total + W - 1) / (uint32_t)W)
@@ -759,13 +824,13 @@ __global__ __launch_bounds__(kStreamWaves * 64, 2) void attn_decode_stream_kerne
 
   // Loop-invariant byte offsets inside a full tile (its base is uniform).
   // K: lane (grp, col) loads key col (+16 for the second half), d 8 grp +
-  // 32 j. V: direct-load instruction i writes LDS rows 4i .. 4i + 3, lane L
-  // row 4i + L / 16 and physical 16-byte chunk L % 16.
-  uint32_t v_off[8];
+  // 32 j. V: direct-load instruction i writes 1 KB of LDS rows, lane L row
+  // (64 i + L) / CPR and physical 16-byte chunk L % CPR.
+  uint32_t v_off[VL];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int r = 4 * i + (lane >> 4), pc = lane & 15;
-    const int chunk = 2 * ((pc >> 1) ^ stream_swizzle(r)) + (pc & 1);
+  for (int i = 0; i < VL; ++i) {
+    const int r = (64 * i + lane) / CPR, pc = lane % CPR;
+    const int chunk = 2 * ((pc >> 1) ^ stream_swizzle<D>(r)) + (pc & 1);
     v_off[i] = (uint32_t)(stream_slot_key(r) * p.v_pos + chunk * 8) * 2u;
   }
   uint32_t k_off[2];
@@ -777,7 +842,7 @@ __global__ __launch_bounds__(kStreamWaves * 64, 2) void attn_decode_stream_kerne
   const int tr_row = 8 * grp + (mu >> 2);
   const int tr_base = tr_row * D + 4 * (mu & 1);
   const int tr_hi = (mu & 3) >> 1;
-  const int tr_f = stream_swizzle(tr_row);
+  const int tr_f = stream_swizzle<D>(tr_row);
 
   // When every key position fits 32 bits (any call below 4 G keys), the
   // divisions of the piece bookkeeping are 32-bit. The lengths come from LDS
@@ -788,25 +853,37 @@ __global__ __launch_bounds__(kStreamWaves * 64, 2) void attn_decode_stream_kerne
   while (pos < end) {
     const uint32_t len_b = s_len[b];
     const uint64_t rel = pos - s_pre[b];
-    const uint32_t j = narrow ? (uint32_t)rel / len_b : (uint32_t)(rel / len_b);  // unit
-    const uint32_t k0 = (uint32_t)(rel - (uint64_t)j * len_b);
-    const uint32_t k1 = (uint32_t)min((uint64_t)len_b, k0 + (end - pos));
+    uint32_t j, k0, k1, first_wg, last_wg;  // unit of the sequence, its keys here, its workgroups
+    if (piece_keys != 0) {
+      const uint32_t np = (len_b + piece_keys - 1) / piece_keys;
+      j = (uint32_t)rel / np;
+      const uint32_t i = (uint32_t)rel - j * np;
+      k0 = i * piece_keys;
+      k1 = min(len_b, k0 + piece_keys);
+      first_wg = w - i;
+      last_wg = first_wg + np - 1;
+    } else {
+      j = narrow ? (uint32_t)rel / len_b : (uint32_t)(rel / len_b);
+      k0 = (uint32_t)(rel - (uint64_t)j * len_b);
+      k1 = (uint32_t)min((uint64_t)len_b, k0 + (end - pos));
+      const uint64_t unit_start = s_pre[b] + (uint64_t)j * len_b;
+      const uint64_t unit_last = unit_start + len_b - 1;
+      first_wg = narrow ? (uint32_t)unit_start / (uint32_t)seg : (uint32_t)(unit_start / seg);
+      last_wg = narrow ? (uint32_t)unit_last / (uint32_t)seg : (uint32_t)(unit_last / seg);
+    }
     const uint32_t kvh = j / p.head_chunks, hc = j % p.head_chunks;
     const uint32_t unit = b * upb + j;
-    const uint64_t unit_start = s_pre[b] + (uint64_t)j * len_b;
-    const uint64_t unit_last = unit_start + len_b - 1;
-    const uint32_t first_wg = narrow ? (uint32_t)unit_start / (uint32_t)seg : (uint32_t)(unit_start / seg);
-    const uint32_t last_wg = narrow ? (uint32_t)unit_last / (uint32_t)seg : (uint32_t)(unit_last / seg);
-    const uint32_t h0 = kvh * p.group + hc * GC;
+    const uint32_t GC = min(p.rows, p.group - hc * p.rows);  // heads of this chunk
+    const uint32_t h0 = kvh * p.group + hc * p.rows;
     uint16_t *out = p.out + (int64_t)b * p.o_seq + (int64_t)h0 * p.o_head;
     const uint32_t ntiles = (k1 - k0 + KT - 1) / KT;
 
     h8_t qop[DC];
     {
-      const uint16_t *qb = p.q + (int64_t)b * p.q_seq + (int64_t)(h0 + min(col, GC - 1)) * p.q_head + 8 * grp;
+      const uint16_t *qb = p.q + (int64_t)b * p.q_seq + (int64_t)(h0 + min((uint32_t)col, GC - 1)) * p.q_head + 8 * grp;
 #pragma unroll
       for (int c = 0; c < DC; ++c)
-        qop[c] = col < GC ? as_h8(*reinterpret_cast<const uint4 *>(qb + 32 * c))
+        qop[c] = (uint32_t)col < GC ? as_h8(*reinterpret_cast<const uint4 *>(qb + 32 * c))
                           : as_h8(make_uint4(0, 0, 0, 0));
     }
     const uint16_t *kb = p.k + (int64_t)b * p.k_seq + (int64_t)kvh * p.k_head;
@@ -829,7 +906,7 @@ __global__ __launch_bounds__(kStreamWaves * 64, 2) void attn_decode_stream_kerne
             kr[hf * DC + c] = load16_stream(reinterpret_cast<const uint16_t *>(kt + k_off[hf] + 64 * c));
         // V is read once too: non-temporal (c4: 111.3 -> 110.1 us, same run).
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
+        for (int i = 0; i < VL; ++i)
           load_lds16_nt(reinterpret_cast<const uint16_t *>(vt + v_off[i]), vdst + i * 512);
       } else {
         // The piece's last, partial tile: rows past it re-read its last key
@@ -842,9 +919,9 @@ __global__ __launch_bounds__(kStreamWaves * 64, 2) void attn_decode_stream_kerne
             kr[hf * DC + c] = load16_stream(kb + (int64_t)key * p.k_pos + 8 * grp + 32 * c);
         }
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int r = 4 * i + (lane >> 4), pc = lane & 15;
-          const int chunk = 2 * ((pc >> 1) ^ stream_swizzle(r)) + (pc & 1);
+        for (int i = 0; i < VL; ++i) {
+          const int r = (64 * i + lane) / CPR, pc = lane % CPR;
+          const int chunk = 2 * ((pc >> 1) ^ stream_swizzle<D>(r)) + (pc & 1);
           const uint32_t key = min(base + (uint32_t)stream_slot_key(r), k1 - 1);
           load_lds16_nt(vb + (int64_t)key * p.v_pos + chunk * 8, vdst + i * 512);
         }
@@ -881,18 +958,23 @@ __global__ __launch_bounds__(kStreamWaves * 64, 2) void attn_decode_stream_kerne
         for (int dt = 0; dt < DB; ++dt) o[dt] *= alpha;
         m_run = m_new;
       }
-      const float mc = m_run == -INFINITY ? 0.0f : m_run * c2;
-      uint32_t pw[4];  // P as f16 pairs in the PV operand's key order
+      const float mc = m_run == -INFINITY ? 0.0f : m_run * c2 - kBias;
+      uint32_t pw[4], pl[4];  // P as f16 pairs in the PV operand's key order (and its low terms)
       float ps = 0.0f;
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
         for (int e = 0; e < 4; e += 2) {
-          const uint32_t wv = pack_f16x2(exp2_raw(fmaf(s[hf][e], c2, -mc)),
-                                           exp2_raw(fmaf(s[hf][e + 1], c2, -mc)));
+          const float p0 = exp2_raw(fmaf(s[hf][e], c2, -mc)), p1 = exp2_raw(fmaf(s[hf][e + 1], c2, -mc));
+          const uint32_t wv = pack_f16x2(p0, p1);
           pw[2 * hf + e / 2] = wv;
-          // The row sum uses the same f16-rounded weights as P V.
-          ps = dot2(wv, 0x3c003c00u, ps);
+          if constexpr (SPLIT_P) {
+            pl[2 * hf + e / 2] = pack_f16x2(p0 - lo_f16(wv), p1 - hi_f16(wv));
+            ps += p0 + p1;
+          } else {
+            // The row sum uses the same f16-rounded weights as P V.
+            ps = dot2(wv, 0x3c003c00u, ps);
+          }
         }
       l_run += ps;
       const h8_t pb = as_h8(make_uint4(pw[0], pw[1], pw[2], pw[3]));
@@ -901,8 +983,11 @@ __global__ __launch_bounds__(kStreamWaves * 64, 2) void attn_decode_stream_kerne
       for (int dt = 0; dt < DB; ++dt) {
         const uint16_t *a0 = vw + tr_base + (2 * (dt ^ tr_f) + tr_hi) * 8;
         const uint2 lo = read_tr16(a0), hi = read_tr16(a0 + 4 * D);
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(make_uint4(lo.x, lo.y, hi.x, hi.y)), pb,
-                                                       o[dt], 0, 0, 0);
+        const h8_t va = as_h8(make_uint4(lo.x, lo.y, hi.x, hi.y));
+        if constexpr (SPLIT_P)
+          o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, as_h8(make_uint4(pl[0], pl[1], pl[2], pl[3])),
+                                                         o[dt], 0, 0, 0);
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pb, o[dt], 0, 0, 0);
       }
     };
 
@@ -924,13 +1009,49 @@ __global__ __launch_bounds__(kStreamWaves * 64, 2) void attn_decode_stream_kerne
     }
     l_run += __shfl_xor(l_run, 16, 64);
     l_run += __shfl_xor(l_run, 32, 64);
+    if constexpr (SPLIT_P) {
+      // An infinite or NaN value row times a zero weight (an empty low term, a
+      // masked re-read key) is NaN in the products above. If any accumulator is
+      // not finite, the wave takes its tiles again on the vector units with
+      // whole f32 weights.
+      float bad = 0.0f;
+#pragma unroll
+      for (int dt = 0; dt < DB; ++dt) bad += (o[dt][0] + o[dt][1] + o[dt][2] + o[dt][3]) * 0.0f;
+      if (__any(!(bad == 0.0f))) {
+        const float mc = m_run == -INFINITY ? 0.0f : m_run * c2 - kBias;
+#pragma unroll
+        for (int dt = 0; dt < DB; ++dt) o[dt] = sf4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (uint32_t t = wave; t < ntiles; t += WAVES)
+          for (uint32_t key = k0 + t * KT; key < min(k1, k0 + (t + 1) * KT); ++key) {
+            const uint16_t *kp = kb + (int64_t)key * p.k_pos, *vp = vb + (int64_t)key * p.v_pos;
+            float sc = 0.0f;
+#pragma unroll
+            for (int c = 0; c < DC; ++c) {
+              const uint4 kv = *reinterpret_cast<const uint4 *>(kp + 8 * grp + 32 * c);
+              const uint4 qv = __builtin_bit_cast(uint4, qop[c]);
+              sc = dot2(qv.x, kv.x, sc);
+              sc = dot2(qv.y, kv.y, sc);
+              sc = dot2(qv.z, kv.z, sc);
+              sc = dot2(qv.w, kv.w, sc);
+            }
+            sc += __shfl_xor(sc, 16, 64);
+            sc += __shfl_xor(sc, 32, 64);
+            const float wgt = exp2_raw(fmaf(sc, c2, -mc));
+#pragma unroll
+            for (int dt = 0; dt < DB; ++dt)
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                o[dt][e] = fmaf(wgt, f16_to_f32(vp[16 * dt + 4 * grp + e]), o[dt][e]);
+          }
+      }
+    }
 
     // Merge the waves through LDS, then write the unit's output (a piece
     // that is the whole unit) or this piece's partial.
     __syncthreads();
     const uint64_t tl_loop_end = tl.clock();
-    float *s_o = reinterpret_cast<float *>(v_lds_a);  // [WAVES][GC][D]
-    if (col < GC) {
+    float *s_o = reinterpret_cast<float *>(v_lds_a);  // [WAVES][GM][D]
+    if ((uint32_t)col < GC) {
       if (grp == 0) {
         s_m[wave][col] = m_run;
         s_l[wave][col] = l_run;
@@ -938,7 +1059,7 @@ __global__ __launch_bounds__(kStreamWaves * 64, 2) void attn_decode_stream_kerne
 #pragma unroll
       for (int dt = 0; dt < DB; ++dt)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s_o[(wave * GC + col) * D + 16 * dt + 4 * grp + e] = o[dt][e];
+        for (int e = 0; e < 4; ++e) s_o[(wave * GM + col) * D + 16 * dt + 4 * grp + e] = o[dt][e];
     }
     __syncthreads();
     const bool direct = first_wg == last_wg;
@@ -948,12 +1069,12 @@ __global__ __launch_bounds__(kStreamWaves * 64, 2) void attn_decode_stream_kerne
     const uint32_t units = p.batch * upb, pieces = last_wg - first_wg + 1;
     const uint32_t S = p.stream_unit_slots;
     const size_t slot = pieces <= S ? (size_t)unit * S + (w - first_wg) : (size_t)units * S + w + unit;
-    float *part = p.partial + slot * GC * (D + 2);
+    float *part = p.partial + slot * p.rows * (D + 2);
     if (w == first_wg && tid == 0)
-      reinterpret_cast<uint32_t *>(p.partial + (size_t)units * (S + 1) * GC * (D + 2) +
-                                   (size_t)p.stream_workgroups * GC * (D + 2))[unit] =
+      reinterpret_cast<uint32_t *>(p.partial + (size_t)units * (S + 1) * p.rows * (D + 2) +
+                                   (size_t)p.stream_workgroups * p.rows * (D + 2))[unit] =
           first_wg | pieces << 16;
-    for (int idx = tid; idx < GC * D; idx += THREADS) {
+    for (int idx = tid; idx < (int)GC * D; idx += THREADS) {
       const int g = idx / D, d = idx % D;
       float M = -INFINITY;
 #pragma unroll
@@ -963,7 +1084,7 @@ __global__ __launch_bounds__(kStreamWaves * 64, 2) void attn_decode_stream_kerne
       for (int wv = 0; wv < WAVES; ++wv) {
         const float f = s_m[wv][g] == -INFINITY ? 0.0f : exp2_raw((s_m[wv][g] - M) * c2);
         L += s_l[wv][g] * f;
-        A += s_o[(wv * GC + g) * D + d] * f;
+        A += s_o[(wv * GM + g) * D + d] * f;
       }
       if (direct) {
         out[g * p.o_head + d] = f32_to_f16(A / L);
@@ -982,7 +1103,7 @@ __global__ __launch_bounds__(kStreamWaves * 64, 2) void attn_decode_stream_kerne
     __syncthreads();
     tl.add(4, 1 | (uint64_t)ntiles << 16);
     tl.add(5, tl.clock() - tl_loop_end);
-    pos += k1 - k0;
+    pos += piece_keys != 0 ? 1 : k1 - k0;
     if (pos < end && pos >= s_pre[b + 1]) b = find_seq(pos);
   }
   tl.now(2);
@@ -1001,28 +1122,23 @@ __global__ __launch_bounds__(kStreamWaves * 64, 2) void attn_decode_stream_kerne
 // against 107.7-107.9 us per call). One thread per output element (GC x 128,
 // at least 256, at most 1024), so the slots load in one pass (c4, GQA 4:
 // 105.7 against 106.0 us with 256 threads and two passes, bit-identical).
-template <int GC>
-constexpr int stream_merge_threads() {
-  return GC * 128 > 1024 ? 1024 : (GC * 128 > 256 ? GC * 128 : 256);
-}
-
-template <int GC>
-__global__ __launch_bounds__(stream_merge_threads<GC>()) void attn_stream_merge_kernel(
-    const RowsParams p) {
-  constexpr int D = 128, THREADS = stream_merge_threads<GC>(), ROW = D + 2;
+template <int D>
+__global__ __launch_bounds__(1024) void attn_stream_merge_kernel(const RowsParams p) {
+  constexpr int ROW = D + 2;
   constexpr int C = kStreamUnitSlots;  // pieces per pass
   const uint32_t S = p.stream_unit_slots;
   const uint32_t upb = p.kv_heads * p.head_chunks;
   const uint32_t unit = blockIdx.x, b = unit / upb, j = unit % upb;
   const uint32_t units = p.batch * upb;
-  const float *own = p.partial + (size_t)unit * S * GC * ROW;
-  const float *overflow = p.partial + (size_t)units * S * GC * ROW;
+  const float *own = p.partial + (size_t)unit * S * p.rows * ROW;
+  const float *overflow = p.partial + (size_t)units * S * p.rows * ROW;
   const uint32_t desc = reinterpret_cast<const uint32_t *>(
-      overflow + (size_t)(p.stream_workgroups + units) * GC * ROW)[unit];
+      overflow + (size_t)(p.stream_workgroups + units) * p.rows * ROW)[unit];
   const uint32_t len_b = min(p.lengths[b], p.kv_length);
   const uint32_t kvh = j / p.head_chunks, hc = j % p.head_chunks;
-  uint16_t *out = p.out + (int64_t)b * p.o_seq + (int64_t)(kvh * p.group + hc * GC) * p.o_head;
-  for (int idx = threadIdx.x; idx < GC * D; idx += THREADS) {
+  const uint32_t GC = min(p.rows, p.group - hc * p.rows);  // heads of this chunk
+  uint16_t *out = p.out + (int64_t)b * p.o_seq + (int64_t)(kvh * p.group + hc * p.rows) * p.o_head;
+  for (uint32_t idx = threadIdx.x; idx < GC * D; idx += blockDim.x) {
     const int g = idx / D, d = idx % D;
     // The unit's own slots, issued before the descriptor is known (in
     // bounds whatever they hold). The compact layout (S = 0) has none: every
@@ -1031,7 +1147,7 @@ __global__ __launch_bounds__(stream_merge_threads<GC>()) void attn_stream_merge_
     if (S != 0) {
 #pragma unroll
       for (int i = 0; i < C; ++i) {
-        const float *ps = own + (size_t)(i * GC + g) * ROW;
+        const float *ps = own + (size_t)(i * p.rows + g) * ROW;
         m[i] = ps[0];
         l[i] = ps[1];
         a[i] = ps[2 + d];
@@ -1040,13 +1156,13 @@ __global__ __launch_bounds__(stream_merge_threads<GC>()) void attn_stream_merge_
     // Zero keys: NaN, written by the stream kernel (the descriptor is stale).
     const uint32_t pieces = desc >> 16;
     if (len_b == 0 || pieces <= 1) return;
-    const float *base = pieces <= S ? own : overflow + (size_t)((desc & 0xffff) + unit) * GC * ROW;
+    const float *base = pieces <= S ? own : overflow + (size_t)((desc & 0xffff) + unit) * p.rows * ROW;
     float M = -INFINITY, Ls = 0.0f, As = 0.0f;
     for (uint32_t s0 = 0; s0 < pieces; s0 += C) {
       if (pieces > S) {
 #pragma unroll
         for (int i = 0; i < C; ++i) {
-          const float *ps = base + (size_t)(min(s0 + i, pieces - 1) * GC + g) * ROW;
+          const float *ps = base + (size_t)(min(s0 + i, pieces - 1) * p.rows + g) * ROW;
           m[i] = ps[0];
           l[i] = ps[1];
           a[i] = ps[2 + d];
@@ -1152,33 +1268,28 @@ hipError_t launch_rows_d(const RowsParams &p, uint32_t waves, uint32_t chunk,
   return hipErrorInvalidValue;
 }
 
-template <int GC>
-hipError_t launch_stream_gc(const RowsParams &p, RowsPhase phase, const Launch &l) {
-  if (phase == RowsPhase::Split)
-    return dispatch(attn_decode_stream_kernel<GC>, dim3(p.stream_workgroups),
-                    dim3(kStreamWaves * 64), 0, l, p);
-  const uint32_t units = p.batch * p.kv_heads * p.head_chunks;
-  return dispatch(attn_stream_merge_kernel<GC>, dim3(units), dim3(stream_merge_threads<GC>()), 0, l,
-                  p);
-}
-
 }  // namespace
 
-uint32_t stream_chunk(uint32_t group) {
-  for (uint32_t c : {16u, 8u, 4u, 2u}) if (group % c == 0) return c;
-  return 1;
+namespace {
+template <int D>
+hipError_t launch_stream_d(const RowsParams &p, RowsPhase phase, const Launch &l) {
+  if (phase == RowsPhase::Split)
+    return dispatch(attn_decode_stream_kernel<D>, dim3(p.stream_workgroups), dim3(kStreamWaves * 64), 0, l, p);
+  const uint32_t units = p.batch * p.kv_heads * p.head_chunks, outs = p.rows * D;
+  return dispatch(attn_stream_merge_kernel<D>, dim3(units), dim3(outs > 1024 ? 1024 : outs > 256 ? outs : 256),
+                  0, l, p);
+}
+}  // namespace
+
+uint32_t stream_workgroups(uint32_t compute_units) {
+  return kStreamPerCu * (compute_units > 1 ? compute_units : 1);
 }
 
-hipError_t launch_decode_stream(const RowsParams &p, uint32_t chunk, RowsPhase phase,
-                                const Launch &l) {
-  switch (chunk) {
-    case 16: return launch_stream_gc<16>(p, phase, l);
-    case 8: return launch_stream_gc<8>(p, phase, l);
-    case 4: return launch_stream_gc<4>(p, phase, l);
-    case 2: return launch_stream_gc<2>(p, phase, l);
-    case 1: return launch_stream_gc<1>(p, phase, l);
-    default: return hipErrorInvalidValue;
-  }
+hipError_t launch_decode_stream(const RowsParams &p, uint32_t head_dim, RowsPhase phase, const Launch &l) {
+  if (p.rows == 0 || p.rows > kDecodeRows) return hipErrorInvalidValue;
+  if (head_dim == 128) return launch_stream_d<128>(p, phase, l);
+  if (head_dim == 64) return launch_stream_d<64>(p, phase, l);
+  return hipErrorInvalidValue;
 }
 
 uint32_t rows_chunk(uint32_t group) {

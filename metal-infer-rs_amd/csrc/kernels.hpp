@@ -193,12 +193,12 @@ constexpr uint32_t kDecodeRows = 16;
 constexpr uint32_t kDecodeWaves = 8;
 hipError_t launch_decode(const RowsParams &p, uint32_t head_dim, const Launch &l);
 
-// Batched decode (one query token per sequence, head_dim 128) on MFMA with
+// Batched decode (one query token per sequence, head_dim 64 or 128) on MFMA with
 // a stream-K split: p.stream_workgroups workgroups share the keys of all
 // sequences equally (each at least kStreamMinKeys). RowsParams as for the
-// rows kernel with tokens = 1, head_chunks = group / chunk and per-sequence
-// `lengths` (required); `partial` holds stream_partial_floats(units,
-// stream_workgroups, chunk, stream_unit_slots) floats: stream_unit_slots
+// rows kernel with tokens = 1, head_chunks chunks of `rows` heads (the last may
+// have fewer) and per-sequence `lengths` (required); with chunk = rows, `partial` holds stream_partial_floats(units,
+// stream_workgroups, chunk, stream_unit_slots, head_dim) floats: stream_unit_slots
 // slots per unit, then stream_workgroups + units overflow slots, each slot
 // chunk * (D + 2) floats, then one u32 descriptor per unit. The Split phase
 // streams the keys and writes units held by one workgroup directly; the
@@ -212,16 +212,15 @@ hipError_t launch_decode(const RowsParams &p, uint32_t head_dim, const Launch &l
 // batch <= kStreamMaxBatch; a full 32-key tile of K or V must span less
 // than 4 GiB (32 * pos stride * 2 bytes).
 constexpr uint32_t kStreamMaxBatch = 1024;
-constexpr uint32_t kStreamMinKeys = 512;
+constexpr uint32_t kStreamMinKeys = 128;
+constexpr uint32_t kStreamPieceMost = 256;  // largest piece of the piece split
 constexpr uint32_t kStreamUnitSlots = 8;
 constexpr uint64_t stream_partial_floats(uint64_t units, uint64_t workgroups, uint32_t chunk,
-                                         uint32_t unit_slots) {
-  return (units * unit_slots + workgroups + units) * chunk * (128 + 2) + units;
+                                         uint32_t unit_slots, uint32_t head_dim) {
+  return (units * unit_slots + workgroups + units) * chunk * (head_dim + 2) + units;
 }
-hipError_t launch_decode_stream(const RowsParams &p, uint32_t chunk, RowsPhase phase,
-                                const Launch &l);
-// Head chunk of the stream kernel: the largest of 16, 8, 4, 2, 1 dividing `group`.
-uint32_t stream_chunk(uint32_t group);
+uint32_t stream_workgroups(uint32_t compute_units);
+hipError_t launch_decode_stream(const RowsParams &p, uint32_t head_dim, RowsPhase phase, const Launch &l);
 
 // Runs rows [row_begin, row_begin + row_count) of the flattened
 // (token, head) grid. Scores of up to kNaiveLdsKeys keys live in LDS; longer

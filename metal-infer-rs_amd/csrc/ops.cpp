@@ -674,6 +674,9 @@ mi_status prepare_qk_norm_rope(mi_batch *batch, const mi_tensor *q, const mi_ten
   return MI_OK;
 }
 
+// Keys per split of the rows kernel's batched decode.
+constexpr uint32_t kRowsBatchedBlock = 768;
+
 // mi_attention_decode_batched with the split partials from `src`.
 mi_status decode_batched(mi_batch *batch, const mi_tensor *q, const mi_tensor *k,
                          const mi_tensor *v, const mi_tensor *lengths,
@@ -729,36 +732,53 @@ mi_status decode_batched(mi_batch *batch, const mi_tensor *q, const mi_tensor *k
   rp.batch = (uint32_t)B, rp.tokens = 1, rp.q_heads = p.Hq, rp.kv_heads = p.Hkv;
   rp.kv_length = p.L, rp.causal = 1, rp.query_offset = 0;
   rp.scale_log2 = (1.0f / std::sqrt((float)p.D)) * 1.4426950408889634f;
-  // Default: the stream-K MFMA kernel (head_dim 128), which gives every
-  // workgroup the same share of all sequences' keys (2 per CU), then its
-  // merge launch. Explicit split sizes keep the rows kernel.
-  if (block_keys == 0 && p.D == 128 && (uint64_t)B <= kernels::kStreamMaxBatch &&
-      pos_stride_fits_u32(k->stride[1], v->stride[1], 32)) {
-    const uint32_t chunk = kernels::stream_chunk(p.G);
-    const uint64_t units = (uint64_t)B * p.Hkv * (p.G / chunk);
-    const uint32_t workgroups = 2 * std::max<uint32_t>(batch->ctx->compute_units, 1);
-    rp.group = p.G, rp.head_chunks = p.G / chunk;
-    rp.stream_workgroups = workgroups;
+  // Default: the stream-K MFMA kernel (head_dim 64 and 128), which gives every
+  // workgroup the same share of all sequences' keys, then its merge launch.
+  // Explicit split sizes keep the rows kernel, and at head_dim 64 so do calls that
+  // it serves in one split without a merge (one sequence of 60 keys 4.4 against
+  // 8.0 us) and few small groups (7 sequences of 16/8 heads 16.0 against 17.0; 20
+  // of them 15.4 against 13.6; 2 of 40/8 heads 12.1 against 11.5).
+  bool stream = block_keys == 0 && (uint64_t)B <= kernels::kStreamMaxBatch &&
+                pos_stride_fits_u32(k->stride[1], v->stride[1], 32) &&
+                (p.D == 128 || (p.D == 64 && p.L > kRowsBatchedBlock &&
+                                (p.G >= 4 || (uint64_t)B * p.Hkv >= 128)));
+  uint64_t bytes = 0;
+  uint32_t unit_slots = 0;
+  if (stream) {
     // Fixed slots per unit, so that the merge loads a unit's pieces with its
     // descriptor; a fixed buffer too small for them takes the compact layout
-    // (every piece in an overflow slot, same merge order and results).
-    uint32_t unit_slots = kernels::kStreamUnitSlots;
-    uint64_t bytes = kernels::stream_partial_floats(units, workgroups, chunk, unit_slots) * sizeof(float);
-    if (src.fixed != nullptr && bytes > src.limit) {
-      unit_slots = 0;
-      bytes = kernels::stream_partial_floats(units, workgroups, chunk, 0) * sizeof(float);
+    // (every piece in an overflow slot, same merge order and results), and then
+    // the largest power-of-two chunks that divide the group, whose overflow
+    // slots are the smallest. At head_dim 64 the rows kernel, whose partials
+    // grow with the capacity instead of the sequences, is left after that.
+    rp.group = p.G, rp.stream_workgroups = kernels::stream_workgroups(batch->ctx->compute_units);
+    for (int attempt = 0; attempt < 3; ++attempt) {
+      rp.head_chunks = std::max(1u, ceil_div(p.G, kernels::kDecodeRows));
+      if (attempt == 2 && p.G != 0)
+        for (rp.head_chunks = 1; p.G % rp.head_chunks != 0 || !pow2(p.G / rp.head_chunks) ||
+                                 p.G / rp.head_chunks > kernels::kDecodeRows;)
+          ++rp.head_chunks;
+      rp.rows = ceil_div(p.G, rp.head_chunks);
+      unit_slots = attempt == 0 ? kernels::kStreamUnitSlots : 0;
+      bytes = kernels::stream_partial_floats((uint64_t)B * p.Hkv * rp.head_chunks, rp.stream_workgroups,
+                                             rp.rows, unit_slots, p.D) *
+              sizeof(float);
+      if (src.fixed == nullptr || bytes <= src.limit) break;
     }
+    if (p.D == 64 && src.fixed != nullptr && bytes > src.limit) stream = false;
+  }
+  if (stream) {
     rp.stream_unit_slots = unit_slots;
     void *scratch = nullptr;
     if ((st = scratch_take(batch, src, bytes, &scratch)) != MI_OK) return st;
     rp.partial = static_cast<float *>(scratch);
     const bool events = src.fixed == nullptr;
     st = launch(batch, "attn_decode_stream", [&](const kernels::Launch &s) {
-      return kernels::launch_decode_stream(rp, chunk, kernels::RowsPhase::Split, s);
+      return kernels::launch_decode_stream(rp, p.D, kernels::RowsPhase::Split, s);
     }, events);
     if (st == MI_OK)
       st = launch(batch, "attn_decode_stream_merge", [&](const kernels::Launch &s) {
-        return kernels::launch_decode_stream(rp, chunk, kernels::RowsPhase::Merge, s);
+        return kernels::launch_decode_stream(rp, p.D, kernels::RowsPhase::Merge, s);
       }, events);
     // In-order execution makes the range reusable by later work of the batch.
     scratch_give(batch->ctx, src, scratch);
@@ -769,7 +789,7 @@ mi_status decode_batched(mi_batch *batch, const mi_tensor *q, const mi_tensor *k
   // Power-of-two splits start every workgroup at the same offset modulo a
   // large power of two, so the workgroups, which stream in lockstep, keep
   // landing on the same HBM channels.
-  if (block_keys == 0) block_keys = std::min<uint32_t>(768, std::max<uint32_t>(64, p.L));
+  if (block_keys == 0) block_keys = std::min<uint32_t>(kRowsBatchedBlock, std::max<uint32_t>(64, p.L));
   if ((st = plan_rows(batch->ctx, &p, (uint64_t)B, p.L, block_keys, 256, true)) != MI_OK)
     return st;
   p.kernel = "attn_rows_batched";

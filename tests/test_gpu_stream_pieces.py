@@ -1,0 +1,79 @@
+"""The batched decode's work split at its edges: pieces of one unit per workgroup (few keys),
+equal segments past them, head groups that are no power of two, and head_dim 64."""
+import numpy as np
+import pytest
+
+import mi_attn
+from helpers import assert_parity, f16, oracle_attention
+
+pytestmark = pytest.mark.gpu
+
+
+def rand(seed, shape, scale=1.0):
+    return (scale * np.random.default_rng(seed).standard_normal(shape)).astype(np.float16).view(np.uint16)
+
+
+def run(ctx, q, k, v, lengths, hq, hkv, d, cap):
+    qt, lt = ctx.tensor(q), ctx.tensor(np.asarray(lengths, np.uint32), mi_attn.U32)
+    kt, vt = (ctx.tensor(np.ascontiguousarray(x.transpose(0, 2, 1, 3))) for x in (k, v))
+    strides = (hkv * cap * d, d, cap * d, 1)
+    kview, vview = kt.view(k.shape, strides), vt.view(v.shape, strides)
+    ctx.take_kernel_profiles()
+    ctx.set_kernel_profiling(True)
+    try:
+        batch = ctx.begin_batch()
+        out = batch.attention_decode_batched(qt, kview, vview, lt, mi_attn.AttentionConfig(hq, hkv, d, True, 0))
+        batch.finish()
+        names = [name for name, _ in ctx.take_kernel_profiles()]
+    finally:
+        ctx.set_kernel_profiling(False)
+    fixed = ctx.empty(q.shape)
+    batch = ctx.begin_batch()
+    batch.attention_decode_batched_noalloc(qt, kview, vview, lt, mi_attn.AttentionConfig(hq, hkv, d, True, 0), 0,
+                                           fixed)
+    batch.finish()
+    got = ctx.download(out)
+    assert (ctx.download(fixed) == got).all()
+    return got, names
+
+
+@pytest.mark.parametrize("hq,hkv,d,cap,lengths", [
+    (16, 8, 128, 1300, [1, 127, 128, 129, 1300]),           # 128-key pieces, more than 8 of a unit
+    (8, 1, 128, 6000, [6000, 0, 5]),                        # 47 pieces of one unit: overflow slots
+    (32, 8, 128, 1100, [256, 257, 512, 1100, 1, 900] * 3),  # 256-key pieces
+    (32, 8, 128, 1200, [1200] * 20),                        # past the pieces: equal segments
+    (40, 8, 128, 500, [500, 33, 64, 0, 499]),               # groups of 5
+    (34, 2, 128, 400, [400, 399]),                          # groups of 17: chunks of 9 and 8
+    (40, 8, 64, 1000, [1000, 33, 64, 0, 999]),
+    (16, 8, 64, 800, [(b * 97) % 801 for b in range(17)]),
+    (64, 8, 64, 3000, [3000, 2999, 1, 768] * 4),
+])
+def test_batched_decode_work_split(ctx, hq, hkv, d, cap, lengths):
+    B = len(lengths)
+    q, k, v = rand(1, (B, hq, d), 2.0), rand(2, (B, cap, hkv, d)), rand(3, (B, cap, hkv, d))
+    got, names = run(ctx, q, k, v, lengths, hq, hkv, d, cap)
+    assert names == ["attn_decode_stream", "attn_decode_stream_merge"], names
+    for b, n in enumerate(lengths):
+        if n == 0:
+            assert np.isnan(f16(got[b])).all()
+            continue
+        ref = oracle_attention(q[b:b + 1], k[b, :n], v[b, :n], hq=hq, hkv=hkv, d=d, off=n - 1)
+        assert_parity(got[b:b + 1], ref, label=f"seq {b} len {n}")
+        if d == 64:  # f32 probabilities: one rounding of the output and a few of the sums
+            bound = np.abs(ref["f32"]) * 2.0 ** -11 + 2.0 ** -24 + 1e-5
+            assert (np.abs(f16(got[b:b + 1]).astype(np.float64) - ref["f32"]) <= bound).all()
+
+
+def test_batched_decode_with_infinite_values_at_head_dim_64(ctx):
+    """An infinite value gives the infinity that the weighted sum gives, in its own column only."""
+    hq, hkv, d, cap, lengths = 32, 8, 64, 800, [800, 37, 300, 65] * 4
+    q, k, v = rand(4, (16, hq, d)), rand(5, (16, cap, hkv, d)), rand(6, (16, cap, hkv, d))
+    for b, n in enumerate(lengths):
+        v[b, n - 1, b % hkv, b] = np.float16(np.inf if b % 2 else -np.inf).view(np.uint16)
+    got, _ = run(ctx, q, k, v, lengths, hq, hkv, d, cap)
+    for b, n in enumerate(lengths):
+        ref = oracle_attention(q[b:b + 1], k[b, :n], v[b, :n], hq=hq, hkv=hkv, d=d, off=n - 1)["f32"]
+        x = f16(got[b:b + 1])
+        assert (np.isposinf(ref) == np.isposinf(x)).all() and (np.isneginf(ref) == np.isneginf(x)).all()
+        fine = np.isfinite(ref)
+        assert np.isfinite(x[fine]).all() and np.abs(x[fine] - ref[fine]).max() <= 2e-3
