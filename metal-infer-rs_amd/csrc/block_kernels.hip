@@ -423,6 +423,83 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(MatvecParams p) {
   }
 }
 
+// Few-row matmul for 2 to kMatvecRows rows of x on MFMA, bound by streaming the
+// weight: one workgroup per FEAT output features, its eight waves on every
+// eighth 256-key chunk of k each. A chunk's weight rows arrive by direct loads of
+// 1 KB (two contiguous 512-byte row pieces) into the wave's own LDS stage,
+// 16-byte piece c of row r at c ^ r, one chunk ahead of the multiply (for k up
+// to 4096 all of the weight is in flight at once), and the x rows straight into
+// the other operand. The waves' sums meet in LDS and add in wave order. FEAT < 16
+// repeats feature rows in the MFMA; it spreads few features over the CUs.
+//
+// The matvec kernel above multiplies every weight piece with every row on the
+// vector units, one load of x for each (MI355X, graph replays over rotated
+// weights, matvec -> this: 8 x [1024, 2048] 7.6 -> 3.8 us, 8 x [4096, 4096] 23.7
+// -> 9.8, 8 x [5120, 8192] 36.5 -> 21.7, 4 x [5120, 5120] 16.5 -> 13.4, 2 x [4096,
+// 4096] 9.2 -> 8.9). One row stays there (7.9 against 8.4 us), and from 9 rows
+// the x operand's loads outweigh the weight's.
+template <int FEAT>
+__global__ __launch_bounds__(512) void stream_matmul_kernel(MatvecParams p) {
+  constexpr int WAVES = 8, CH = kStreamMatmulChunk, STEPS = CH / 32;
+  constexpr int LOADS = FEAT * CH * 2 / 1024, CPR = CH / 8;  // 1 KB loads per chunk, 16-byte pieces per row
+  constexpr int STAGE = FEAT * CH;
+  typedef float sf4 __attribute__((ext_vector_type(4)));
+  __shared__ __attribute__((aligned(16))) uint16_t s_a[WAVES * STAGE], s_b[WAVES * STAGE];
+  __shared__ __attribute__((aligned(16))) float s_acc[WAVES][64][4];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const uint32_t n0 = blockIdx.x * FEAT;
+  const uint32_t chunks = p.k / CH;
+  const uint16_t *src[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int row = (64 * i + lane) / CPR;
+    src[i] = p.w + (int64_t)min(n0 + row, p.n - 1) * p.w_row + 8 * ((lane % CPR) ^ (row & 15));
+  }
+  const int r = lane & 15, kg = lane >> 4;
+  const uint16_t *xr = p.x + (int64_t)min((uint32_t)r, p.m - 1) * p.x_row + 8 * kg;
+  int at[STEPS];
+#pragma unroll
+  for (int s = 0; s < STEPS; ++s) at[s] = wave * STAGE + (r % FEAT) * CH + (((4 * s + kg) ^ (r % FEAT)) * 8);
+  uint4 xa[STEPS], xb[STEPS];
+  auto issue = [&](uint32_t c, uint16_t *dst, uint4 *xv) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) load_lds16_nt(src[i] + (size_t)c * CH, dst + wave * STAGE + i * 512);
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) xv[s] = load16(xr + (size_t)c * CH + 32 * s);
+  };
+  sf4 acc = sf4{0.0f, 0.0f, 0.0f, 0.0f};
+  auto compute = [&](const uint16_t *lds, const uint4 *xv) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+      const h8_t a = as_h8(*reinterpret_cast<const uint4 *>(lds + at[s]));
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, as_h8(xv[s]), acc, 0, 0, 0);
+    }
+  };
+  uint32_t c = wave;
+  if (c < chunks) issue(c, s_a, xa);
+  while (c < chunks) {
+    uint32_t nx = c + WAVES;
+    if (nx < chunks) issue(nx, s_b, xb);
+    compute(s_a, xa);
+    c = nx;
+    if (c >= chunks) break;
+    nx = c + WAVES;
+    if (nx < chunks) issue(nx, s_a, xa);
+    compute(s_b, xb);
+    c = nx;
+  }
+  *reinterpret_cast<sf4 *>(s_acc[wave][lane]) = acc;
+  __syncthreads();
+  // Lane (row, kg) of a wave holds features 4 kg .. 4 kg + 3 of that row of x.
+  if (tid < 16 * FEAT) {
+    const int f = tid % FEAT, row = tid / FEAT;
+    float v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) v += s_acc[w][(f >> 2) * 16 + row][f & 3];
+    if ((uint32_t)row < p.m && n0 + f < p.n) p.out[(int64_t)row * p.o_row + n0 + f] = f32_to_f16(v);
+  }
+}
+
 // Few-row matmul (the decode o_proj, matvec_f16 family of
 // transformer.metal:274-400): one wave per weight row (= output column),
 // four per workgroup. Lanes stream the row in 16-byte pieces (64 lanes cover
@@ -560,6 +637,24 @@ hipError_t launch_skinny_gemm(const MatvecParams &p, uint32_t compute_units, con
   if (!skinny_gemm_supported(p, compute_units)) return hipErrorInvalidValue;
   if (p.m <= 16) return dispatch(skinny_gemm_kernel<1>, dim3(p.n / 16), dim3(256), 0, l, p);
   return dispatch(skinny_gemm_kernel<2>, dim3(p.n / 16), dim3(256), 0, l, p);
+}
+
+bool stream_matmul_supported(const MatvecParams &p) {
+  return p.m > 1 && p.m <= kMatvecRows && p.n > 0 && p.k > 0 && p.k % kStreamMatmulChunk == 0 &&
+         p.x_row % 8 == 0 && p.w_row % 8 == 0 && aligned16(p.x) && aligned16(p.w);
+}
+
+hipError_t launch_stream_matmul(const MatvecParams &p, uint32_t compute_units, const Launch &l) {
+  if (!stream_matmul_supported(p)) return hipErrorInvalidValue;
+  // The most features per workgroup that still give every CU one; past 16 per
+  // CU, 8 with two workgroups per CU (8 x [5120, 8192]: 21.7 against 24.7 us).
+  auto run = [&](auto feat_tag) {
+    constexpr int FEAT = decltype(feat_tag)::value;
+    return dispatch(stream_matmul_kernel<FEAT>, dim3((p.n + FEAT - 1) / FEAT), dim3(512), 0, l, p);
+  };
+  if (p.n <= 4ull * compute_units) return run(std::integral_constant<int, 4>{});
+  if (p.n > 8ull * compute_units && p.n <= 16ull * compute_units) return run(std::integral_constant<int, 16>{});
+  return run(std::integral_constant<int, 8>{});
 }
 
 hipError_t launch_matvec(const MatvecParams &p, const Launch &l) {

@@ -264,6 +264,10 @@ mi_status mi_matmul(mi_batch *batch, const mi_tensor *input, const mi_tensor *we
   // grid fits the device; it measured 9.9 us against hipBLASLt's 12.1 us for
   // [32, 4096] x [4096, 4096]^T.
   const uint32_t cus = batch->ctx->compute_units;
+  if (kernels::stream_matmul_supported(p))
+    return launch(batch, "stream_matmul", [&](const kernels::Launch &l) {
+      return kernels::launch_stream_matmul(p, cus, l);
+    });
   if (kernels::skinny_gemm_supported(p, cus))
     return launch(batch, "skinny_gemm",
                   [&](const kernels::Launch &l) { return kernels::launch_skinny_gemm(p, cus, l); });

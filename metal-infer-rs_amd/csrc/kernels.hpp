@@ -273,6 +273,11 @@ struct MatvecParams {
   uint32_t m, n, k;
 };
 constexpr uint32_t kMatvecRows = 8;
+// Two to kMatvecRows rows on MFMA: k % kStreamMatmulChunk == 0 and x, w rows
+// 16-byte aligned.
+constexpr uint32_t kStreamMatmulChunk = 256;
+bool stream_matmul_supported(const MatvecParams &p);
+hipError_t launch_stream_matmul(const MatvecParams &p, uint32_t compute_units, const Launch &l);
 // Skinny GEMM for kMatvecRows < m <= kSkinnyMaxRows, bound by streaming the
 // weight: one workgroup per 16 output features. Requires n % 16 == 0 with
 // n / 16 at most the device's CUs, k % (8 * kSkinnyChunkSteps * 64) == 0 and

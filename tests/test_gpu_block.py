@@ -307,6 +307,25 @@ def test_rms_norm_parity(ctx, shape):
     check_rms_norm(got, x, w, 1e-6, str(shape))
 
 
+@pytest.mark.parametrize("n", [4, 1023, 1024, 1030, 4096, 4100])
+@pytest.mark.parametrize("m,k", [(2, 256), (8, 2048), (7, 2304), (3, 4352)])
+def test_matmul_few_rows_on_mfma(ctx, m, n, k):
+    """Two to eight rows: every feature count per workgroup with a part-filled last one, fewer
+    chunks of k than waves, one and more per wave; strided x rows."""
+    x, w = rand(m + n, (m, k + 8)), rand(k, (n, k), scale=k ** -0.5)
+    dev = ctx.tensor(x)
+    out = ctx.empty((m, n + 2))
+    batch = ctx.begin_batch()
+    batch.matmul(dev.view((m, k), (k + 8, 1)), ctx.tensor(w), out=out.view((m, n), (n + 2, 1)))
+    batch.finish()
+    exact = f16(x[:, :k]).astype(np.float64) @ f16(w).astype(np.float64).T
+    terms = np.abs(f16(x[:, :k])).astype(np.float64) @ np.abs(f16(w)).astype(np.float64).T
+    # One rounding of the output; f32 sums of k products in eight parts.
+    bound = np.abs(exact) * 2.0 ** -11 + terms * (k / 8 + 16) * 2.0 ** -24 + 2.0 ** -24
+    got = f16(ctx.download(out))[:, :n]
+    assert (np.abs(got - exact) <= bound).all()
+
+
 @pytest.mark.parametrize("width", [64, 128, 256])
 @pytest.mark.parametrize("rows", [1, 33, 4 * 32 * 2 * 256 + 5])
 def test_rms_norm_narrow_rows(ctx, width, rows):
