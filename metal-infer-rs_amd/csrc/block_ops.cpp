@@ -271,6 +271,10 @@ mi_status mi_matmul(mi_batch *batch, const mi_tensor *input, const mi_tensor *we
   if (kernels::skinny_gemm_supported(p, cus))
     return launch(batch, "skinny_gemm",
                   [&](const kernels::Launch &l) { return kernels::launch_skinny_gemm(p, cus, l); });
+  // More rows, as long as one output tile per CU covers them.
+  if (kernels::gemm_tile_supported(p, cus))
+    return launch(batch, "gemm",
+                  [&](const kernels::Launch &l) { return kernels::launch_gemm_tile(p, cus, l); });
   // Empty products (n or k of 0) stay on the few-row kernel: no launch for
   // n == 0, zeros for k == 0.
   if (p.m > kernels::kMatvecRows && p.n > 0 && p.k > 0) {

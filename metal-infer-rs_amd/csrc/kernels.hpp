@@ -286,6 +286,11 @@ constexpr uint32_t kSkinnyMaxRows = 32;
 constexpr uint32_t kSkinnyChunkSteps = 2;  // 64-key steps per LDS chunk
 bool skinny_gemm_supported(const MatvecParams &p, uint32_t compute_units);
 hipError_t launch_skinny_gemm(const MatvecParams &p, uint32_t compute_units, const Launch &l);
+// More rows than the skinny GEMM's, one output tile per CU (gemm_tile.hip): its
+// tiles fit the device's CUs at once and measured faster, k % 128 == 0, n % 4 == 0, x and w rows
+// 16-byte and out rows 8-byte aligned.
+bool gemm_tile_supported(const MatvecParams &p, uint32_t compute_units);
+hipError_t launch_gemm_tile(const MatvecParams &p, uint32_t compute_units, const Launch &l);
 
 hipError_t launch_rms_norm(const RmsNormParams &p, uint32_t compute_units, const Launch &l);
 hipError_t launch_rope(const RopeParams &p, const Launch &l);
