@@ -415,10 +415,11 @@ mi_status mi_rope(mi_batch *batch, const mi_tensor *input, uint64_t offset,
                   float theta, const mi_tensor *out);
 /* CommandBatch::matmul (ops.rs:242-373): out[m, n] = f16(sum_k input[m, k] *
  * weight[n, k]) with f32 accumulation (weight in the checkpoint's
- * [out_features, in_features] layout). Up to 8 rows run the library's
- * HBM-streaming few-row kernel; more rows run a hipBLASLt f16 GEMM with f32
- * compute, planned once per shape (or the few-row kernel over groups of 8
- * rows when hipBLASLt has no solution for the shape). */
+ * [out_features, in_features] layout). Up to 32 rows run the library's
+ * weight-streaming kernels; more rows run its tile GEMM as far as one output
+ * tile per CU covers them, else (and for layouts those kernels do not read) a
+ * hipBLASLt f16 GEMM with f32 compute, planned once per shape (or the few-row
+ * kernel over groups of 8 rows when hipBLASLt has no solution for the shape). */
 mi_status mi_matmul(mi_batch *batch, const mi_tensor *input,
                     const mi_tensor *weight, const mi_tensor *out);
 

@@ -547,9 +547,10 @@ def test_captured_unfused_decode_step_replays_match_eager(ctx):
     cache.close()
 
 
-def test_captured_gemm_replays_match_eager(ctx):
-    """A prefill-sized o_proj (hipBLASLt) recorded into a graph."""
-    m, n, k = 64, 1024, 2048
+@pytest.mark.parametrize("m,n,k", [(64, 1024, 2048), (64, 1024, 2080)])
+def test_captured_gemm_replays_match_eager(ctx, m, n, k):
+    """A prefill-sized o_proj recorded into a graph: the tile GEMM, and hipBLASLt
+    for a k that is no multiple of 128."""
     x = ctx.tensor(rand(110, (m, k)))
     w = ctx.tensor(rand(111, (n, k), scale=k ** -0.5))
     out = ctx.empty((m, n))
