@@ -234,8 +234,12 @@ mi_status mi_context_synchronize(mi_context *ctx);
 /* set_kernel_profiling / take_kernel_profiles (context.rs:602-700): when
  * enabled, every kernel a batch launches carries start / stop HIP events
  * bound to its dispatch (hipExtLaunchKernelGGL), and its execution time is
- * reported per launch after wait. A split-K attention records its split
- * pass ("attn_rows") and merge pass ("attn_merge") separately. */
+ * reported per launch after wait. Names tell the kernels apart ("attn_rows",
+ * "attn_decode", "attn_tiled", "attn_prefill", "attn_decode_stream"; the decode
+ * step "attn_decode_step" or "attn_decode_step_mfma"; matmul "matvec",
+ * "stream_matmul", "skinny_gemm", "gemm_tile" or the library's "gemm"), and
+ * a merge launch is a record of its own ("attn_merge", "attn_tiled_merge",
+ * "attn_decode_stream_merge"). */
 mi_status mi_context_set_kernel_profiling(mi_context *ctx, int32_t enabled);
 mi_status mi_context_take_kernel_profiles(mi_context *ctx,
                                           mi_kernel_profile *out,

@@ -273,7 +273,7 @@ mi_status mi_matmul(mi_batch *batch, const mi_tensor *input, const mi_tensor *we
                   [&](const kernels::Launch &l) { return kernels::launch_skinny_gemm(p, cus, l); });
   // More rows, as long as one output tile per CU covers them.
   if (kernels::gemm_tile_supported(p, cus))
-    return launch(batch, "gemm",
+    return launch(batch, "gemm_tile",
                   [&](const kernels::Launch &l) { return kernels::launch_gemm_tile(p, cus, l); });
   // Empty products (n or k of 0) stay on the few-row kernel: no launch for
   // n == 0, zeros for k == 0.

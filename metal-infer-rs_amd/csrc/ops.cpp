@@ -168,7 +168,7 @@ bool plan_decode(const Context *ctx, AttnPlan *p, uint32_t max_keys, bool step) 
   const uint32_t splits = (uint32_t)std::max<uint64_t>(
       1, std::min<uint64_t>(ceil_div(max_keys, 128), cus / units));
   p->family = Family::Decode;
-  p->kernel = "attn_rows";
+  p->kernel = "attn_decode";
   p->waves = kernels::kDecodeWaves;
   p->threads = p->waves * 64;
   p->block_keys = ceil_div(ceil_div(max_keys, splits), 32) * 32;
@@ -1136,7 +1136,7 @@ mi_status mi_decode_step_attention(mi_batch *batch, const mi_tensor *q, const mi
   rp.step_kc = static_cast<uint16_t *>(key_cache->data);
   rp.step_vc = static_cast<uint16_t *>(value_cache->data);
   rp.step_theta = qp.theta, rp.step_eps = qp.epsilon;
-  p.kernel = "attn_decode_step";
+  p.kernel = p.family == Family::Decode ? "attn_decode_step_mfma" : "attn_decode_step";
   return run_rows(batch, p, rp);
 }
 

@@ -194,20 +194,20 @@ def test_matmul_skinny_views(ctx, pad, offset):
     check_matmul(ctx.download(out), rows, w, f"view pad={pad} offset={offset}")
 
 
-@pytest.mark.parametrize("m,n,k,pad", [
-    (33, 4, 128, 0),        # one step, one tile with four features
-    (64, 100, 256, 8),      # 32 x 32, fewer steps than stages, padded rows
-    (65, 1028, 896, 0),     # 32 x 32, seven steps
-    (300, 1024, 640, 0),    # 64 x 32
-    (257, 2052, 1664, 8),   # 64 x 64, 13 steps
-    (1100, 1020, 384, 0),   # 64 x 96, three steps
-    (1537, 1024, 512, 4),   # 128 x 64, 13 row tiles: a band of 8 and one of 5; x rows 8 bytes off: library
-    (1537, 1020, 512, 0),
-    (1101, 2048, 128, 0),   # 192 x 64, two steps
-    (1101, 2044, 576, 0),   # k no multiple of 128: library
-    (40, 5120, 5120, 0),    # narrow tiles, long rows: library
+@pytest.mark.parametrize("m,n,k,pad,kernel", [
+    (33, 4, 128, 0, "gemm_tile"),        # one step, one tile with four features
+    (64, 100, 256, 8, "gemm_tile"),      # 32 x 32, fewer steps than stages, padded rows
+    (65, 1028, 896, 0, "gemm_tile"),     # 32 x 32, seven steps
+    (300, 1024, 640, 0, "gemm_tile"),    # 64 x 32
+    (257, 2052, 1664, 8, "gemm_tile"),   # 64 x 64, 13 steps
+    (1100, 1020, 384, 0, "gemm_tile"),   # 64 x 96, three steps
+    (1537, 1024, 512, 4, "gemm"),        # x rows 8 bytes off: library
+    (1537, 1020, 512, 0, "gemm_tile"),   # 128 x 64, 13 row tiles: a band of 8 and one of 5
+    (1101, 2048, 128, 0, "gemm_tile"),   # 192 x 64, two steps
+    (1101, 2044, 576, 0, "gemm"),        # k no multiple of 128: library
+    (40, 5120, 5120, 0, "gemm"),         # narrow tiles, long rows: library
 ])
-def test_matmul_tiled_rows(ctx, m, n, k, pad):
+def test_matmul_tiled_rows(ctx, m, n, k, pad, kernel):
     """More than 32 rows: one output tile per CU, at each tile's remainders, and
     the calls beside it that stay on the library; the same bits when repeated."""
     x_store = rand(500 + m, (m, k + pad))
@@ -219,9 +219,13 @@ def test_matmul_tiled_rows(ctx, m, n, k, pad):
     got = []
     for _ in range(2):
         ctx.upload(out, np.full((m, n + pad), 0x7e00, np.uint16))
+        ctx.take_kernel_profiles()
+        ctx.set_kernel_profiling(True)
         batch = ctx.begin_batch()
         batch.matmul(x_view, w_dev, out=rows)
         batch.finish()
+        ctx.set_kernel_profiling(False)
+        assert [name for name, _ in ctx.take_kernel_profiles()] == [kernel]
         got.append(ctx.download(out))
     assert (got[0] == got[1]).all()
     assert (got[0][:, n:] == 0x7e00).all()

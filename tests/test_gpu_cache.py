@@ -290,15 +290,15 @@ def test_captured_fused_decode_step_replays_match_eager(ctx, one_launch):
 
 # ------------------------------------------- one-launch decode attention step --
 
-@pytest.mark.parametrize("hq,hkv,d,pos", [
-    (16, 8, 128, 2047),   # c2: 16 splits merged in the launch
-    (32, 8, 128, 300),    # GQA 4
-    (64, 8, 128, 100),    # GQA 8, one split
-    (16, 8, 128, 0),      # the new token is the only key
-    (8, 8, 128, 1000),    # MHA
-    (8, 4, 64, 500),      # head_dim 64: the three calls' kernels
+@pytest.mark.parametrize("hq,hkv,d,pos,kernels", [
+    (16, 8, 128, 2047, ["attn_decode_step"]),       # c2: 16 splits merged in the launch
+    (32, 8, 128, 300, ["attn_decode_step"]),        # GQA 4
+    (64, 8, 128, 100, ["attn_decode_step_mfma"]),   # GQA 8, one split
+    (16, 8, 128, 0, ["attn_decode_step"]),          # the new token is the only key
+    (8, 8, 128, 1000, ["attn_decode_step"]),        # MHA
+    (8, 4, 64, 500, ["qk_norm_rope_cache", "attn_decode"]),  # head_dim 64: the three calls' kernels
 ])
-def test_decode_step_matches_the_three_calls(ctx, hq, hkv, d, pos):
+def test_decode_step_matches_the_three_calls(ctx, hq, hkv, d, pos, kernels):
     """mi_decode_step_attention == qk_norm_rope_cache_value then FlashDecode
     over the prefix [0, pos] (qwen3.rs:704-750), and both match the oracle."""
     cap, theta, eps = pos + 3, 1_000_000.0, 1e-6
@@ -331,8 +331,7 @@ def test_decode_step_matches_the_three_calls(ctx, hq, hkv, d, pos):
         finally:
             ctx.set_kernel_profiling(False)
         if fused:
-            want = ["attn_decode_step"] if d == 128 else ["qk_norm_rope_cache", "attn_rows"]
-            assert names[:len(want)] == want, names
+            assert names == kernels, names
         results.append((ctx.download(out), ctx.download(key), ctx.download(value)))
         cache.close()
     (out_pair, key_pair, value_pair), (out_step, key_step, value_step) = results

@@ -40,7 +40,7 @@ def test_few_row_attention(ctx, hq, hkv, d, T, off, extra, causal, kind):
     info = ctx.plan(qt, kview, kview, mi_attn.AttentionConfig(hq, hkv, d, causal, off), KINDS[kind])
     group, chunks = hq // hkv, 1 if T > 1 else -(-hq // hkv // 16)
     rows = T * -(-group // chunks)
-    assert info["block_threads"] == 512 and info["grid"][1] == hkv * chunks, info
+    assert info["kernel"] == "attn_decode" and info["block_threads"] == 512 and info["grid"][1] == hkv * chunks, info
     assert info["scratch_bytes"] in (0, info["grid"][1] * info["splits"] * rows * (d + 2) * 4), info
     out = run_attention(ctx, q, k, v, kind=kind, layout="position_major", **geo)
     again = run_attention(ctx, q, k, v, kind=kind, layout="head_major", **geo)
@@ -69,8 +69,8 @@ def test_few_row_attention_with_infinite_values(ctx, d, T, off, kind):
     assert np.isfinite(got[fine]).all() and np.abs(got[fine] - ref[fine]).max() <= 2e-3
 
 
-@pytest.mark.parametrize("hq,hkv,pos", [(64, 8, 0), (64, 8, 32), (8, 1, 300), (40, 2, 129), (32, 8, 3500),
-                                        (17, 1, 900)])
+@pytest.mark.parametrize("hq,hkv,pos", [(64, 8, 0), (64, 8, 32), (8, 1, 300), (40, 2, 1700), (32, 8, 3500),
+                                        (17, 1, 9000)])
 def test_decode_step_on_the_mfma_kernel(ctx, hq, hkv, pos):
     """The one-launch step: no cached key, splits and head chunks; the cache row that it writes is
     the only one that changes, and what the row held before has no influence."""
@@ -84,10 +84,14 @@ def test_decode_step_on_the_mfma_kernel(ctx, hq, hkv, pos):
     ctx.upload(key, hist_k)
     ctx.upload(value, hist_v)
     tensors = [ctx.tensor(x) for x in (q, k, v, qw, kw)]
+    ctx.take_kernel_profiles()
+    ctx.set_kernel_profiling(True)
     batch = ctx.begin_batch()
     out = batch.decode_step_attention(*tensors, key, value, mi_attn.QkNormRopeCacheConfig(pos, 1e6, 1e-6),
                                       mi_attn.AttentionConfig(hq, hkv, d, True, pos))
     batch.finish()
+    ctx.set_kernel_profiling(False)
+    assert [name for name, _ in ctx.take_kernel_profiles()] == ["attn_decode_step_mfma"]
     got, key_now, value_now = ctx.download(out), ctx.download(key), ctx.download(value)
     others = np.arange(cap) != pos
     assert (key_now[others] == hist_k[others]).all() and (value_now[others] == hist_v[others]).all()
