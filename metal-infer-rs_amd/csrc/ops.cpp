@@ -131,34 +131,55 @@ mi_status plan_rows(const Context *ctx, AttnPlan *p, uint64_t batch, uint32_t ma
   return MI_OK;
 }
 
-// Whether the few-row MFMA kernel (attn_decode.hip) is the faster one for T tokens
-// over `keys` keys. The rows kernel spends vector arithmetic on every (row, key),
-// and one workgroup of it on every head chunk and token; the MFMA kernel has the
-// longer fixed chain. Measured on MI355X (graph replays, rotated caches; rows /
-// MFMA us): 8-head chunks 64/8 heads at 300 keys 13.3 / 9.6, 100 keys 10.0 / 5.2;
-// 4-head chunks, one or two tokens, 32/8 at 100 keys 6.4 / 5.2, 1000 keys 9.2 /
-// 9.0, 2 x 500 10.7 / 9.8. Smaller chunks cross at a number of (row, key) pairs
-// that grows with the rows to merge: 16/8 at 4095 keys 9.3 / 9.5, 5000 11.5 /
-// 10.3; 40/8 (five one-head chunks) at 1000 7.8 / 9.4, 2000 10.9 / 9.9; 2 tokens
-// of 16/8 at 1500 8.5 / 9.3, 3000 9.9 / 9.7; 4 of 32/8 at 1500 12.3 / 13.0, 6000
-// 25.4 / 15.7. At head_dim 64 the fixed chain is shorter: 16/8 at 300 to 2000
-// keys 6.6-7.1 / 6.6-7.0, 32/8 at 300 8.9 / 6.7, 40/8 at 400 6.0 / 7.3. The
-// decode step's transforms lengthen the chain, so its 4-head chunks cross later
-// (32/8 at 2000 keys 10.7 / 10.9; 64/8 at 300 15.5 / 11.2).
-bool decode_mfma_wins(const AttnPlan &p, uint64_t keys, bool step) {
-  const uint32_t chunk = kernels::rows_chunk(p.G), rows = p.T * p.G;
-  if (p.T <= 2 && chunk >= (p.D == 64 ? 2u : step ? 8u : 4u)) return true;
-  const uint64_t cross = 6144 + 1280 * (uint64_t)rows;
-  return rows * keys >= (p.D == 64 ? cross / 2 : cross);
+// Whether the few-row MFMA kernel (attn_decode.hip), which would run `rows` packed
+// rows in `splits` splits per unit, is the faster one for T tokens over `keys`
+// keys. The rows kernel spends vector arithmetic on every (row, key), in chunks of
+// 8, 4, 2 or 1 heads that each read K/V again; the MFMA kernel has the longer fixed
+// chain, and its last workgroup merges `splits * rows` partial rows. So the lines
+// lie where the heads make a chunk of 4 or 8, or where the (row, key) pairs per CU
+// outweigh that chain, and end where the merge does. Measured on MI355X (graph
+// replays over rotated caches, 24 head geometries from 2/1 to 128/8 by 18 lengths
+// from 17 to 32768 keys, one token and 2 to 16 rows; rows / MFMA us): within 2% of
+// the faster one or better wherever this says true.
+//  - One token, chunks of 4 and 8: 64/8 heads at 300 keys 14.4 / 10.5, 20000 keys
+//    31.9 / 22.2; 32/8 at 300 9.6 / 9.4. More than 8 rows (groups past 8): 16/1 at
+//    9000 keys 22.7 / 22.9, at 20000 (157 splits) 31.0 / 33.0.
+//  - One token, groups of 2: at head_dim 64 from the first key on (16/8 at 300
+//    7.0 / 6.9); at 128 16/8 at 3000 9.1 / 9.7, 4500 11.1 / 10.5, 20000 19.9 /
+//    20.4; never in the decode step, whose transforms lengthen the chain (16/8 at
+//    4500 11.5 / 12.4, 12000 14.6 / 16.9). Groups of 1: never (8/8 at 12000 keys
+//    14.4 / 15.3).
+//  - One token, groups in several chunks of 1 or 2: 7/1 at 12000 keys 9.2 / 14.3,
+//    20/4 at 6000 11.5 / 11.7, 9000 25.7 / 12.6, 40/8 at 4500 26.6 / 11.7; 48/8
+//    (chunks of 2) at 1500 9.7 / 10.4, 2000 12.5 / 10.3.
+//  - Several tokens: chunks of 8 always (64/8, 2 tokens on 300 keys 14.7 / 12.0);
+//    2 tokens of a group of 4 (at head_dim 64 of 2) from 32 keys (32/8 at 130
+//    9.8 / 8.9); else 8/8, 8 tokens at 1000 keys 9.4 / 10.1, 3000 16.9 / 10.8; 2/1,
+//    8 tokens at 12000 13.7 / 23.3; 28/4, 2 tokens at 1000 9.4 / 11.9, 2200 18.0 /
+//    12.5.
+bool decode_mfma_wins(const AttnPlan &p, uint64_t keys, bool step, uint64_t rows, uint64_t splits,
+                      uint64_t cus) {
+  const uint32_t chunk = kernels::rows_chunk(p.G), chunks = p.G / chunk;
+  const uint64_t merge = splits * rows, pairs = (uint64_t)p.T * p.Hq * keys / cus;
+  if (p.T == 1) {
+    if (chunk >= 4) return rows <= 8 || merge <= (step ? 512 : 1536);
+    if (chunks > 1) return pairs >= (chunk == 2 ? 375 : 562) && merge <= 1024;
+    if (chunk == 1) return false;
+    return p.D == 64 || (!step && pairs >= 256 && pairs <= 1000 && merge <= 512);
+  }
+  if (chunk == 8) return merge <= 1536;
+  if (p.T == 2 && chunks == 1 && chunk >= (p.D == 64 ? 2u : 4u)) return keys >= 32 && merge <= 1024;
+  if (chunks > 1 && p.Hkv >= 4) return pairs >= 375 && merge <= 1024;
+  return pairs >= 750 && merge <= (chunk == 1 ? 1024 : 512);
 }
 
-// The few-row MFMA kernel's plan: about one 8-wave workgroup per CU, each with at
-// least 128 keys (half its waves busy: 192 or 256 measured slower at every
-// length, 2047 keys 9.3 against 8.7 us). False if it cannot or should not run.
+// The few-row MFMA kernel's plan: about one 8-wave workgroup per CU, the keys in as
+// many equal splits (a multiple of 32 keys) as there are whole or started pieces
+// of 128 keys (half the waves of one busy: pieces of 192 or 256 measured slower at
+// every length, 2047 keys 9.3 against 8.7 us). False if it cannot or should not run.
 bool plan_decode(const Context *ctx, AttnPlan *p, uint32_t max_keys, bool step) {
   if ((p->D != 64 && p->D != 128) || p->T == 0 || p->G == 0 || max_keys == 0) return false;
   if (p->T > 1 && (uint64_t)p->T * p->G > kernels::kDecodeRows) return false;
-  if (!decode_mfma_wins(*p, max_keys, step)) return false;
   const uint32_t chunks = p->T == 1 ? ceil_div(p->G, kernels::kDecodeRows) : 1;
   const uint32_t rows = ceil_div(p->G, chunks) * p->T;
   const uint64_t units = (uint64_t)p->Hkv * chunks;
@@ -167,12 +188,14 @@ bool plan_decode(const Context *ctx, AttnPlan *p, uint32_t max_keys, bool step) 
   const uint64_t cus = std::max<uint32_t>(ctx ? ctx->compute_units : 256, 1);
   const uint32_t splits = (uint32_t)std::max<uint64_t>(
       1, std::min<uint64_t>(ceil_div(max_keys, 128), cus / units));
+  const uint32_t block_keys = ceil_div(ceil_div(max_keys, splits), 32) * 32;
+  if (!decode_mfma_wins(*p, max_keys, step, rows, ceil_div(max_keys, block_keys), cus)) return false;
   p->family = Family::Decode;
   p->kernel = "attn_decode";
   p->waves = kernels::kDecodeWaves;
   p->threads = p->waves * 64;
-  p->block_keys = ceil_div(ceil_div(max_keys, splits), 32) * 32;
-  p->splits = ceil_div(max_keys, p->block_keys);
+  p->block_keys = block_keys;
+  p->splits = ceil_div(max_keys, block_keys);
   p->fused = true;
   p->chunk = rows;
   p->head_chunks = chunks;
@@ -289,14 +312,19 @@ void order_prefill_pieces(const Context *ctx, AttnPlan *p, bool causal, uint32_t
 // at least two tiles where the row tiles do not fill the chip (two workgroups per
 // CU measured the same with twice the partials; fewer than 8 key tiles are not
 // split, 200 tokens of 32/8 heads alone 10.8 against 13.2 us). The rows kernel
-// reads every key again for every token; small calls are still faster on it
-// (measured on MI355X, rows / this: 16/8 heads, 10 tokens on 300 keys 8.3 / 10.6
-// us, 32/8, 10 on 500 13.7 / 10.1, 64/8, 4 on 2000 19.9 / 13.0, 32/8, 24 on 6000
-// 108 / 20, 16/8, 2000 alone 473 / 55).
+// reads every key again for every token, in head chunks; small calls are still
+// faster on it. With chunks of 4 and 8 heads the line is 12000 (row, key) pairs per
+// KV head (32/8 heads, 10 tokens on 500 keys 13.7 / 10.1 us, rows / this; 64/8, 4
+// on 2000 19.9 / 13.0; 32/8, 24 on 6000 108 / 20). With chunks of 1 and 2 it spreads
+// over the chip better than one workgroup per row tile: unsplit, this takes a
+// time by key tiles (8/8, 40 tokens on 300 keys, 6 tiles, 8.6 / 13.4; 16/8, 128
+// alone, 2 tiles, 7.2 / 7.8; 40/8, 64 alone, one tile, 9.8 / 6.4), split, the
+// two launches (8/8, 8 tokens on 1500 keys 11.0 / 11.4, 16 on 1500 16.5 / 11.4;
+// 7/1, 4 on 6000 at head_dim 64 12.6 / 13.7).
 bool plan_tiled(const Context *ctx, AttnPlan *p, uint32_t max_keys) {
   if ((p->D != 64 && p->D != 128) || p->T <= 1 || p->G == 0 || max_keys == 0) return false;
   const uint64_t rows = (uint64_t)p->T * p->G;
-  if (rows >= (1ull << 31) || rows * max_keys < 12000) return false;
+  if (rows >= (1ull << 31)) return false;
   const uint64_t cus = std::max<uint32_t>(ctx ? ctx->compute_units : 256, 1);
   const uint32_t row_tiles = ceil_div(rows, kernels::kPrefillBlockM);
   if (row_tiles > 0xffffu || p->Hkv > 0xffffu) return false;
@@ -305,6 +333,11 @@ bool plan_tiled(const Context *ctx, AttnPlan *p, uint32_t max_keys) {
   const uint32_t want =
       tiles < 8 ? 1 : (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(tiles / 2, cus / wgs));
   const uint32_t per_split = ceil_div(tiles, want);
+  const uint64_t pairs = rows * p->Hkv * max_keys / cus;
+  if (rows * max_keys < 12000) return false;
+  const uint32_t chunk = kernels::rows_chunk(p->G);
+  const uint64_t line = per_split < tiles ? (p->Hkv == 1 ? 1376 : 688) : (chunk == 2 ? 344 : 250) * (1ull + tiles);
+  if (chunk < 4 && pairs < line) return false;
   p->family = Family::Tiled;
   p->kernel = "attn_tiled";
   p->threads = 256;

@@ -151,6 +151,42 @@ def test_flash_decode_accepts_every_gqa_ratio():
         assert p["grid"][1] == hkv * (group // chunk)  # each KV row read once per chunk
 
 
+@pytest.mark.parametrize("hq,hkv,d,T,L,kind,kernel", [
+    # One token: groups whose heads make no chunk of 4 or 8, on either side of the line.
+    (7, 1, 128, 1, 12000, DECODE_SPLIT_KV, "attn_rows"),
+    (28, 4, 64, 1, 1500, DECODE_SPLIT_KV, "attn_rows"),
+    (28, 4, 128, 1, 9000, DECODE_SPLIT_KV, "attn_decode"),
+    (40, 8, 128, 1, 4500, DECODE_SPLIT_KV, "attn_decode"),
+    (48, 8, 64, 1, 1500, DECODE_SPLIT_KV, "attn_rows"),
+    (8, 8, 128, 1, 12000, DECODE_SPLIT_KV, "attn_rows"),
+    (32, 32, 64, 1, 32768, DECODE_SPLIT_KV, "attn_rows"),
+    (16, 8, 128, 1, 3000, DECODE_SPLIT_KV, "attn_rows"),
+    (16, 8, 128, 1, 6000, DECODE_SPLIT_KV, "attn_decode"),
+    (16, 8, 128, 1, 32768, DECODE_SPLIT_KV, "attn_rows"),
+    (16, 8, 64, 1, 300, DECODE_SPLIT_KV, "attn_decode"),
+    (16, 1, 128, 1, 9000, DECODE_SPLIT_KV, "attn_decode"),
+    (16, 1, 128, 1, 20000, DECODE_SPLIT_KV, "attn_rows"),  # 157 splits of 16 rows to merge
+    # Up to 16 rows of several tokens.
+    (2, 1, 128, 8, 12008, TILED, "attn_rows"),
+    (16, 8, 128, 8, 3008, TILED, "attn_decode"),
+    (14, 2, 64, 2, 4502, TILED, "attn_rows"),
+    (64, 8, 128, 2, 302, TILED, "attn_decode"),
+    # More rows: the rows kernel's workgroups against one per row tile.
+    (8, 8, 128, 40, 340, TILED, "attn_rows"),
+    (16, 8, 64, 64, 364, TILED, "attn_rows"),
+    (7, 1, 64, 3, 6003, TILED, "attn_rows"),
+    (8, 8, 64, 128, 428, TILED, "attn_rows"),
+    (8, 8, 128, 128, 828, TILED, "attn_tiled"),
+    (40, 8, 128, 64, 64, TILED, "attn_tiled"),
+    (32, 8, 128, 10, 500, TILED, "attn_tiled"),
+])
+def test_attention_routes_at_the_measured_lines(hq, hkv, d, T, L, kind, kernel):
+    """The rows kernel and the MFMA kernels, each where it measured faster on 256 CUs (what a plan
+    without a context assumes)."""
+    q, k = tensor((T, hq, d)), tensor((L, hkv, d))
+    assert plan(q, k, k, AttentionConfig(hq, hkv, d, True, L - T), kind)["kernel"] == kernel
+
+
 def test_causal_window_bounds_the_splits():
     # Keys past query_offset are never visited: 65 keys, offset 62 -> 63 visible.
     q, k, v = tensor((1, 16, 128)), tensor((65, 8, 128)), tensor((65, 8, 128))

@@ -292,7 +292,7 @@ def test_captured_fused_decode_step_replays_match_eager(ctx, one_launch):
 
 @pytest.mark.parametrize("hq,hkv,d,pos,kernels", [
     (16, 8, 128, 2047, ["attn_decode_step"]),       # c2: 16 splits merged in the launch
-    (32, 8, 128, 300, ["attn_decode_step"]),        # GQA 4
+    (32, 8, 128, 300, ["attn_decode_step_mfma"]),   # GQA 4
     (64, 8, 128, 100, ["attn_decode_step_mfma"]),   # GQA 8, one split
     (16, 8, 128, 0, ["attn_decode_step"]),          # the new token is the only key
     (8, 8, 128, 1000, ["attn_decode_step"]),        # MHA

@@ -22,13 +22,13 @@ def rand(seed, shape, scale=1.0):
     (32, 8, 128, 1, 99, 57, False, "flash-decode"),    # non-causal: every key
     (64, 8, 128, 1, 4999, 0, True, "flash-decode"),    # 32 splits: a whole merge pass
     (8, 1, 128, 1, 9000, 0, True, "flash-decode"),     # 71 splits: three merge passes
-    (17, 1, 128, 1, 2300, 0, True, "flash-decode"),    # two head chunks of 9 and 8
+    (17, 1, 128, 1, 9000, 0, True, "flash-decode"),    # two head chunks of 9 and 8
     (40, 2, 64, 1, 777, 0, True, "decode-split-kv"),   # two head chunks of 10
     (32, 8, 64, 1, 300, 0, True, "flash-decode"),
     (16, 8, 64, 1, 5000, 0, True, "flash-decode"),
     (32, 8, 128, 2, 30, 0, True, "tiled"),             # two tokens, windows across a tile edge
     (32, 8, 128, 4, 3001, 0, True, "tiled"),           # 16 rows
-    (15, 3, 128, 3, 4000, 5, True, "tiled"),           # 15 rows of 5 heads
+    (15, 3, 128, 3, 4400, 5, True, "tiled"),           # 15 rows of 5 heads
     (16, 8, 64, 8, 1900, 0, False, "tiled"),
     (12, 1, 64, 1, 2047, 0, True, "tiled"),
 ])
