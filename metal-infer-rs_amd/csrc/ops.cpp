@@ -150,27 +150,37 @@ mi_status plan_rows(const Context *ctx, AttnPlan *p, uint64_t batch, uint32_t ma
 //    4500 11.5 / 12.4, 12000 14.6 / 16.9). Groups of 1: never (8/8 at 12000 keys
 //    14.4 / 15.3).
 //  - One token, groups in several chunks of 1 or 2: 7/1 at 12000 keys 9.2 / 14.3,
-//    20/4 at 6000 11.5 / 11.7, 9000 25.7 / 12.6, 40/8 at 4500 26.6 / 11.7; 48/8
-//    (chunks of 2) at 1500 9.7 / 10.4, 2000 12.5 / 10.3.
+//    20/4 at 6000 11.5 / 11.7, 9000 25.7 / 12.6; with 8 KV heads from 2000 keys
+//    (24/8 at 1500 8.5 / 9.7, 2000 11.3 / 9.7; 48/8, chunks of 2, 9.7 / 10.4,
+//    12.5 / 10.3; 40/8 at 4500 26.6 / 11.7).
 //  - Several tokens: chunks of 8 always (64/8, 2 tokens on 300 keys 14.7 / 12.0);
-//    2 tokens of a group of 4 (at head_dim 64 of 2) from 32 keys (32/8 at 130
-//    9.8 / 8.9); else 8/8, 8 tokens at 1000 keys 9.4 / 10.1, 3000 16.9 / 10.8; 2/1,
-//    8 tokens at 12000 13.7 / 23.3; 28/4, 2 tokens at 1000 9.4 / 11.9, 2200 18.0 /
-//    12.5.
+//    2 tokens of a group of 4, at head_dim 128 from 32 keys, at 64 also of 2 (32/8
+//    at 130 9.8 / 8.9); else by pairs, and by keys where KV heads or head chunks
+//    alone make the rows kernel's workgroups many: 8/8, 8 tokens at 1000 keys 9.4 / 10.1, 3000 16.9 / 10.8, 3 at
+//    1500 8.8 / 9.0, 2200 10.0 / 9.1; 14/2, 2 tokens at 4500 16.7 / 17.5, 12000
+//    30.0 / 23.3; 2/1, 8 tokens at 12000 13.7 / 23.3; 28/4, 2 tokens at 1000
+//    9.4 / 11.9, 2200 18.0 / 12.5.
 bool decode_mfma_wins(const AttnPlan &p, uint64_t keys, bool step, uint64_t rows, uint64_t splits,
                       uint64_t cus) {
   const uint32_t chunk = kernels::rows_chunk(p.G), chunks = p.G / chunk;
   const uint64_t merge = splits * rows, pairs = (uint64_t)p.T * p.Hq * keys / cus;
   if (p.T == 1) {
-    if (chunk >= 4) return rows <= 8 || merge <= (step ? 512 : 1536);
-    if (chunks > 1) return pairs >= (chunk == 2 ? 375 : 562) && merge <= 1024;
+    if (chunk >= 4) return rows <= 8 || merge <= (step && keys < 9000 ? 512 : 1536);
+    if (chunks > 1)
+      return ((p.Hkv >= 8 && keys >= 2000) || pairs >= (chunk == 2 ? 375 : 562)) && merge <= 1024;
     if (chunk == 1) return false;
     return p.D == 64 || (!step && pairs >= 256 && pairs <= 1000 && merge <= 512);
   }
   if (chunk == 8) return merge <= 1536;
-  if (p.T == 2 && chunks == 1 && chunk >= (p.D == 64 ? 2u : 4u)) return keys >= 32 && merge <= 1024;
-  if (chunks > 1 && p.Hkv >= 4) return pairs >= 375 && merge <= 1024;
-  return pairs >= 750 && merge <= (chunk == 1 ? 1024 : 512);
+  if (p.T == 2 && chunks == 1 && chunk >= (p.D == 64 ? 2u : 4u))
+    return (p.D == 64 || keys >= 32) && merge <= 1024;
+  if (merge > (p.Hkv == 1 ? 512 : 1536)) return false;
+  uint64_t line = 750;
+  if (chunks > 1 && p.Hkv >= 4)
+    line = keys >= 2200 ? 0 : keys >= 1500 ? 280 : 375;
+  else if (keys >= (p.Hkv >= 32 ? 1000 : p.Hkv >= 16 ? 1500 : 2200))
+    line = p.Hkv >= 8 ? 0 : p.Hkv >= 4 ? 450 : p.Hkv >= 2 ? 530 : 750;
+  return pairs >= line;
 }
 
 // The few-row MFMA kernel's plan: about one 8-wave workgroup per CU, the keys in as
@@ -307,24 +317,43 @@ void order_prefill_pieces(const Context *ctx, AttnPlan *p, bool causal, uint32_t
   p->grid[2] = 1;
 }
 
+// The (row, key) pairs per CU from which the Tiled kind's MFMA kernel
+// (attn_tiled.hip) with these key tiles and splits beats the rows kernel, which
+// reads every key again for every token and head chunk but spreads over the chip
+// better than one workgroup per row tile. Measured on MI355X (graph replays, 24 head
+// geometries, 2 to 600 tokens on 0 to 6000 cached keys; rows / this us). Chunks of 8,
+// and of 4 with several KV heads: no line (32/8 heads, 10 tokens on 500 keys 13.7 /
+// 10.1; 64/8, 4 on 2000 19.9 / 13.0; 32/8, 24 on 6000 108 / 20). Else, unsplit, this
+// takes a time by key tiles (8/8, 40 tokens on 300 keys, 6 tiles, 8.6 / 13.4, 200
+// alone, 4 tiles, 9.7 / 10.6; 16/8, 128 alone, 2 tiles, 7.2 / 7.8; 40/8, 64 alone, one
+// tile, 9.8 / 6.4; 4/1, 64 on 300 11.8 / 13.7, on 100 9.6 / 6.7), and split, that of two
+// launches and of the partials (8/8, 8 tokens on 1500 keys 11.0 / 11.4, 16 16.5 /
+// 11.4; 16/8, 5 on 1500 10.7 / 11.6; 28/4, 3 on 700 9.2 / 10.6, 4 on 1500 19.2 / 11.0;
+// 6/2, 5 on 3000 8.5 / 10.2; past 32 splits 7/1, 4 on 6000 at head_dim 64 12.6 /
+// 13.7; 4/1, 16 on 6000 12.1 / 14.1, 40 on 3000 24.6 / 13.7).
+uint64_t tiled_line(const AttnPlan &p, uint64_t tiles, uint32_t splits) {
+  const uint32_t chunk = kernels::rows_chunk(p.G);
+  const bool many = p.G > chunk;  // several chunks per group
+  if (chunk >= 4) {
+    if (chunk == 8 || p.Hkv > 1) return 0;
+    if (splits > 1) return splits > 32 ? 1800 : 900;
+    return tiles < 6 ? 0 : 60 * (1 + 2 * tiles);
+  }
+  if (splits > 32) return 900;
+  if (splits > 1) return many && p.Hkv >= 4 ? 280 : chunk == 2 ? 600 : 400;
+  return (many ? 104 : chunk == 2 ? 205 : 142) * (1 + 2 * tiles);
+}
+
 // The Tiled kind's MFMA plan for more rows than the few-row kernel takes (or fewer
 // where that one loses): about one workgroup per CU, the keys split into ranges of
 // at least two tiles where the row tiles do not fill the chip (two workgroups per
 // CU measured the same with twice the partials; fewer than 8 key tiles are not
-// split, 200 tokens of 32/8 heads alone 10.8 against 13.2 us). The rows kernel
-// reads every key again for every token, in head chunks; small calls are still
-// faster on it. With chunks of 4 and 8 heads the line is 12000 (row, key) pairs per
-// KV head (32/8 heads, 10 tokens on 500 keys 13.7 / 10.1 us, rows / this; 64/8, 4
-// on 2000 19.9 / 13.0; 32/8, 24 on 6000 108 / 20). With chunks of 1 and 2 it spreads
-// over the chip better than one workgroup per row tile: unsplit, this takes a
-// time by key tiles (8/8, 40 tokens on 300 keys, 6 tiles, 8.6 / 13.4; 16/8, 128
-// alone, 2 tiles, 7.2 / 7.8; 40/8, 64 alone, one tile, 9.8 / 6.4), split, the
-// two launches (8/8, 8 tokens on 1500 keys 11.0 / 11.4, 16 on 1500 16.5 / 11.4;
-// 7/1, 4 on 6000 at head_dim 64 12.6 / 13.7).
+// split, 200 tokens of 32/8 heads alone 10.8 against 13.2 us). Below 12000 pairs per
+// KV head the rows kernel is the faster one for every group.
 bool plan_tiled(const Context *ctx, AttnPlan *p, uint32_t max_keys) {
   if ((p->D != 64 && p->D != 128) || p->T <= 1 || p->G == 0 || max_keys == 0) return false;
   const uint64_t rows = (uint64_t)p->T * p->G;
-  if (rows >= (1ull << 31)) return false;
+  if (rows >= (1ull << 31) || rows * max_keys < 12000) return false;
   const uint64_t cus = std::max<uint32_t>(ctx ? ctx->compute_units : 256, 1);
   const uint32_t row_tiles = ceil_div(rows, kernels::kPrefillBlockM);
   if (row_tiles > 0xffffu || p->Hkv > 0xffffu) return false;
@@ -333,15 +362,12 @@ bool plan_tiled(const Context *ctx, AttnPlan *p, uint32_t max_keys) {
   const uint32_t want =
       tiles < 8 ? 1 : (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(tiles / 2, cus / wgs));
   const uint32_t per_split = ceil_div(tiles, want);
-  const uint64_t pairs = rows * p->Hkv * max_keys / cus;
-  if (rows * max_keys < 12000) return false;
-  const uint32_t chunk = kernels::rows_chunk(p->G);
-  const uint64_t line = per_split < tiles ? (p->Hkv == 1 ? 1376 : 688) : (chunk == 2 ? 344 : 250) * (1ull + tiles);
-  if (chunk < 4 && pairs < line) return false;
+  const uint32_t splits = ceil_div(tiles, per_split);
+  if (rows * p->Hkv * max_keys / cus < tiled_line(*p, tiles, splits)) return false;
   p->family = Family::Tiled;
   p->kernel = "attn_tiled";
   p->threads = 256;
-  p->splits = ceil_div(tiles, per_split);
+  p->splits = splits;
   p->block_keys = p->splits > 1 ? per_split * kernels::kPrefillBlockN : 0;
   p->grid[0] = p->splits;
   p->grid[1] = row_tiles;

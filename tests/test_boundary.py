@@ -144,11 +144,13 @@ def test_flash_decode_accepts_every_gqa_ratio():
     for hq, hkv in ((16, 8), (32, 8), (64, 8), (8, 8), (24, 8)):
         q, k, v, cfg = _decode(hq, hkv)
         p = plan(q, k, v, cfg, FLASH_DECODE)
+        # K/V rows are read once per KV head on the MFMA kernel (groups of 4 and 8, and of 3
+        # from 2000 keys on), once per head chunk on the rows kernel.
         group = hq // hkv
-        # The plan names the kernel that runs: the MFMA one for groups of 4 and 8.
-        assert p["kernel"] == ("attn_decode" if group % 4 == 0 else "attn_rows")
+        mfma = group in (3, 4, 8)
+        assert p["kernel"] == ("attn_decode" if mfma else "attn_rows")
         chunk = max(c for c in (8, 4, 2, 1) if group % c == 0)
-        assert p["grid"][1] == hkv * (group // chunk)  # each KV row read once per chunk
+        assert p["grid"][1] == (hkv if mfma else hkv * (group // chunk))
 
 
 @pytest.mark.parametrize("hq,hkv,d,T,L,kind,kernel", [
@@ -169,7 +171,8 @@ def test_flash_decode_accepts_every_gqa_ratio():
     # Up to 16 rows of several tokens.
     (2, 1, 128, 8, 12008, TILED, "attn_rows"),
     (16, 8, 128, 8, 3008, TILED, "attn_decode"),
-    (14, 2, 64, 2, 4502, TILED, "attn_rows"),
+    (6, 2, 64, 3, 303, TILED, "attn_rows"),
+    (14, 2, 64, 2, 12002, TILED, "attn_decode"),
     (64, 8, 128, 2, 302, TILED, "attn_decode"),
     # More rows: the rows kernel's workgroups against one per row tile.
     (8, 8, 128, 40, 340, TILED, "attn_rows"),
