@@ -32,6 +32,7 @@
 // than four in two (32768 keys: 31 against 42 us: half the partials to merge).
 #include <type_traits>
 
+#include "decode_tile.hpp"
 #include "device_common.hpp"
 #include "kernels.hpp"
 
@@ -43,31 +44,12 @@ using namespace mi::dev;
 
 typedef float f4_t __attribute__((ext_vector_type(4)));
 
-constexpr int KT = 32;  // keys per wave tile
+constexpr int KT = kDecodeTile;
 // The exponent added to every probability: 2^(s - m_ref + kBias), so that the
 // low f16 term of a weight of 2^-8 of the largest still has 22 bits above
 // f16's smallest value. With the lazy rescale below a weight is at most
 // 2^(kBias + 8).
 constexpr float kBias = 6.0f;
-
-__device__ __forceinline__ uint4 load16_nt(const uint16_t *ptr) {
-  typedef unsigned u4_t __attribute__((ext_vector_type(4)));
-  const u4_t x = __builtin_nontemporal_load(reinterpret_cast<const u4_t *>(ptr));
-  return make_uint4(x.x, x.y, x.z, x.w);
-}
-
-// Key of LDS row r of a V tile: k-slot 8 g + i of the PV operand holds key
-// 16 (i / 4) + 4 g + i % 4, the keys lane group g holds in the S accumulator.
-__device__ __forceinline__ int slot_key(int r) {
-  return (((r >> 2) & 1) << 4) | (((r >> 3) & 3) << 2) | (r & 3);
-}
-// XOR applied to the 32-byte column pair of V row r, so that the 16 rows of one
-// transposed read fall on all 8 bank groups twice. D = 64: rows are half a
-// bank row, so their parity already picks one of two halves.
-template <int D>
-__device__ __forceinline__ int v_swizzle(int r) {
-  return D == 128 ? ((r & 3) | (((r >> 3) & 1) << 2)) : (((r >> 1) & 1) | (((r >> 3) & 1) << 1));
-}
 
 // Wave slots of the workgroup merge: one per wave, and one for the new token of
 // a decode step.
@@ -142,8 +124,8 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void attn_decode_kernel(const
 #pragma unroll
   for (int i = 0; i < VL; ++i) {
     const int r = (64 * i + lane) / CPR, pc = lane % CPR;
-    const int chunk = 2 * ((pc >> 1) ^ v_swizzle<D>(r)) + (pc & 1);
-    v_off[i] = (uint32_t)(slot_key(r) * p.v_pos + chunk * 8) * 2u;
+    const int chunk = 2 * ((pc >> 1) ^ decode_v_swizzle<D>(r)) + (pc & 1);
+    v_off[i] = (uint32_t)(decode_slot_key(r) * p.v_pos + chunk * 8) * 2u;
   }
 #pragma unroll
   for (int hf = 0; hf < 2; ++hf) k_off[hf] = (uint32_t)((16 * hf + col) * p.k_pos + 8 * grp) * 2u;
@@ -174,8 +156,8 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void attn_decode_kernel(const
 #pragma unroll
       for (int i = 0; i < VL; ++i) {
         const int r = (64 * i + lane) / CPR, pc = lane % CPR;
-        const int chunk = 2 * ((pc >> 1) ^ v_swizzle<D>(r)) + (pc & 1);
-        const uint32_t key = min(base + (uint32_t)slot_key(r), k1 - 1);
+        const int chunk = 2 * ((pc >> 1) ^ decode_v_swizzle<D>(r)) + (pc & 1);
+        const uint32_t key = min(base + (uint32_t)decode_slot_key(r), k1 - 1);
         load_lds16_nt(vb + (int64_t)key * p.v_pos + chunk * 8, vdst + i * 512);
       }
     }
@@ -305,13 +287,14 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void attn_decode_kernel(const
   // d 16 dt + 4 (mu % 4).
   const int tr_row = 8 * grp + (col >> 2);
   const int tr_base = tr_row * D + 4 * (col & 1);
-  const int tr_hi = (col & 3) >> 1, tr_f = v_swizzle<D>(tr_row);
+  const int tr_hi = (col & 3) >> 1, tr_f = decode_v_swizzle<D>(tr_row);
   f4_t o[DB];
 #pragma unroll
   for (int dt = 0; dt < DB; ++dt) o[dt] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
   float m_run = -INFINITY, l_run = 0.0f;  // raw-score reference max, row sum
 
-  auto compute = [&](uint32_t ti, const uint4 *kr, const uint16_t *vst) __attribute__((always_inline)) {
+  // `finite` is a constant of the main loop: every value of the tile is.
+  auto compute = [&](uint32_t ti, const uint4 *kr, const uint16_t *vst, bool finite) __attribute__((always_inline)) {
     const uint32_t base = k0 + ti * KT;
     f4_t s[2];  // s[hf][e]: row col, key 16 hf + 4 grp + e
 #pragma unroll
@@ -344,6 +327,17 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void attn_decode_kernel(const
       m_run = m_new;
     }
     const float mc = m_run == -INFINITY ? 0.0f : m_run * c2 - kBias;
+    if (!finite) {
+      float w[2][4];
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[hf][e] = exp2_raw(fmaf(s[hf][e], c2, -mc));
+      const uint32_t lim = min(k1, vis);
+      weigh_tile<D>(o, w, vst + wave * STAGE, v_lds_b + wave * STAGE, grp, col,
+                    lim > base ? (int)min(lim - base, (uint32_t)KT) : 0);
+      return;
+    }
     // P as f16 pairs in the PV operand's key order: hi, and what it rounded off.
     uint32_t ph[4], pl[4];
     float ps = 0.0f;
@@ -374,12 +368,12 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void attn_decode_kernel(const
   while (ti < ntiles) {
     uint32_t nx = ti + WAVES;
     if (nx < ntiles) issue(nx, krb, v_lds_b);
-    compute(ti, kra, v_lds_a);
+    compute(ti, kra, v_lds_a, true);
     ti = nx;
     if (ti >= ntiles) break;
     nx = ti + WAVES;
     if (nx < ntiles) issue(nx, kra, v_lds_a);
-    compute(ti, krb, v_lds_b);
+    compute(ti, krb, v_lds_b, true);
     ti = nx;
   }
   l_run += __shfl_xor(l_run, 16, 64);
@@ -387,38 +381,23 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void attn_decode_kernel(const
 
   // An infinite or NaN value row times a zero weight (a masked key, an empty low
   // term) is NaN in the products above. If any accumulator is not finite, the
-  // wave takes its tiles again on the vector units, visible keys only and with
-  // whole f32 weights.
+  // wave takes its tiles again, those that hold such a value on the vector units
+  // (visible keys only, whole f32 weights).
   {
     float bad = 0.0f;
 #pragma unroll
     for (int dt = 0; dt < DB; ++dt) bad += (o[dt][0] + o[dt][1] + o[dt][2] + o[dt][3]) * 0.0f;
     if (__any(!(bad == 0.0f))) {
-      const float mc = m_run == -INFINITY ? 0.0f : m_run * c2 - kBias;
+      const float l_sum = l_run;
 #pragma unroll
       for (int dt = 0; dt < DB; ++dt) o[dt] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-      for (uint32_t t = wave; t < ntiles; t += WAVES)
-        for (uint32_t key = k0 + t * KT; key < min(k1, k0 + (t + 1) * KT); ++key) {
-          const uint16_t *kp = kb + (int64_t)key * p.k_pos, *vp = vb + (int64_t)key * p.v_pos;
-          float sc = 0.0f;
-#pragma unroll
-          for (int j = 0; j < DC; ++j) {
-            const uint4 kv = *reinterpret_cast<const uint4 *>(kp + 8 * grp + 32 * j);
-            sc = dot2(qraw[j].x, kv.x, sc);
-            sc = dot2(qraw[j].y, kv.y, sc);
-            sc = dot2(qraw[j].z, kv.z, sc);
-            sc = dot2(qraw[j].w, kv.w, sc);
-          }
-          sc += __shfl_xor(sc, 16, 64);
-          sc += __shfl_xor(sc, 32, 64);
-          if (key >= vis) continue;
-          const float w = exp2_raw(fmaf(sc, c2, -mc));
-#pragma unroll
-          for (int dt = 0; dt < DB; ++dt)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              o[dt][e] = fmaf(w, f16_to_f32(vp[16 * dt + 4 * grp + e]), o[dt][e]);
-        }
+#pragma unroll 1
+      for (uint32_t t = wave; t < ntiles; t += WAVES) {
+        issue(t, kra, v_lds_a);
+        __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+        compute(t, kra, v_lds_a, !any_not_finite<2 * STAGE>(v_lds_a + wave * STAGE, lane));
+      }
+      l_run = l_sum;
     }
   }
 

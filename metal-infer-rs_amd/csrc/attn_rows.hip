@@ -22,6 +22,7 @@
 // (attn_decode_stream_kernel: MFMA tiles, stream-K split).
 #include <type_traits>
 
+#include "decode_tile.hpp"
 #include "device_common.hpp"
 #include "kernels.hpp"
 #include "timeline.hpp"
@@ -646,31 +647,12 @@ __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(
 //  - The 4 waves take interleaved tiles, each with two register / LDS stages
 //    (the next tile is in flight while one is computed).
 constexpr int kStreamWaves = 4;
-constexpr int kStreamTile = 32;
 
 #ifdef MI_TIMELINE
 __device__ uint64_t stream_timeline[kTimelineSlots * kTimelineFields];
 #endif
 
 typedef float sf4_t __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ uint4 load16_stream(const uint16_t *ptr) {
-  typedef unsigned u4_t __attribute__((ext_vector_type(4)));
-  const u4_t x = __builtin_nontemporal_load(reinterpret_cast<const u4_t *>(ptr));
-  return make_uint4(x.x, x.y, x.z, x.w);
-}
-// Key of LDS row r of a V tile: k-slot 8 g + i of the PV operand holds key
-// 16 (i / 4) + 4 g + i % 4, the keys lane group g holds in the S accumulator.
-__device__ __forceinline__ int stream_slot_key(int r) {
-  return (((r >> 2) & 1) << 4) | (((r >> 3) & 3) << 2) | (r & 3);
-}
-// XOR applied to the 32-byte column pair of V row r: the 16 rows of one
-// transposed read then fall on 8 distinct bank groups (D = 64: rows are half a
-// bank row, so their parity already picks one of two halves).
-template <int D>
-__device__ __forceinline__ int stream_swizzle(int r) {
-  return D == 128 ? ((r & 3) | (((r >> 3) & 1) << 2)) : (((r >> 1) & 1) | (((r >> 3) & 1) << 1));
-}
 
 // Workgroups per CU of the stream kernel's launch (three at D = 64 measured
 // slower: 32 sequences of 1024 to 8192 keys 64.7 against 60.6 us).
@@ -685,7 +667,7 @@ constexpr int kStreamPerCu = 2;
 template <int D>
 __global__ __launch_bounds__(kStreamWaves * 64, kStreamPerCu) void attn_decode_stream_kernel(
     const RowsParams p) {
-  constexpr int WAVES = kStreamWaves, KT = kStreamTile, DC = D / 32, DB = D / 16;
+  constexpr int WAVES = kStreamWaves, KT = kDecodeTile, DC = D / 32, DB = D / 16;
   constexpr int CPR = D / 8, VL = KT * CPR / 64;  // 16-byte chunks per V row, 1 KB V loads per tile
   constexpr bool SPLIT_P = D == 64;
   // Added to every weight's exponent, so that low terms stay above f16's
@@ -830,8 +812,8 @@ __global__ __launch_bounds__(kStreamWaves * 64, kStreamPerCu) void attn_decode_s
 #pragma unroll
   for (int i = 0; i < VL; ++i) {
     const int r = (64 * i + lane) / CPR, pc = lane % CPR;
-    const int chunk = 2 * ((pc >> 1) ^ stream_swizzle<D>(r)) + (pc & 1);
-    v_off[i] = (uint32_t)(stream_slot_key(r) * p.v_pos + chunk * 8) * 2u;
+    const int chunk = 2 * ((pc >> 1) ^ decode_v_swizzle<D>(r)) + (pc & 1);
+    v_off[i] = (uint32_t)(decode_slot_key(r) * p.v_pos + chunk * 8) * 2u;
   }
   uint32_t k_off[2];
 #pragma unroll
@@ -842,7 +824,7 @@ __global__ __launch_bounds__(kStreamWaves * 64, kStreamPerCu) void attn_decode_s
   const int tr_row = 8 * grp + (mu >> 2);
   const int tr_base = tr_row * D + 4 * (mu & 1);
   const int tr_hi = (mu & 3) >> 1;
-  const int tr_f = stream_swizzle<D>(tr_row);
+  const int tr_f = decode_v_swizzle<D>(tr_row);
 
   // When every key position fits 32 bits (any call below 4 G keys), the
   // divisions of the piece bookkeeping are 32-bit. The lengths come from LDS
@@ -903,7 +885,7 @@ __global__ __launch_bounds__(kStreamWaves * 64, kStreamPerCu) void attn_decode_s
         for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
           for (int c = 0; c < DC; ++c)
-            kr[hf * DC + c] = load16_stream(reinterpret_cast<const uint16_t *>(kt + k_off[hf] + 64 * c));
+            kr[hf * DC + c] = load16_nt(reinterpret_cast<const uint16_t *>(kt + k_off[hf] + 64 * c));
         // V is read once too: non-temporal (c4: 111.3 -> 110.1 us, same run).
 #pragma unroll
         for (int i = 0; i < VL; ++i)
@@ -916,18 +898,19 @@ __global__ __launch_bounds__(kStreamWaves * 64, kStreamPerCu) void attn_decode_s
           const uint32_t key = min(base + 16 * hf + col, k1 - 1);
 #pragma unroll
           for (int c = 0; c < DC; ++c)
-            kr[hf * DC + c] = load16_stream(kb + (int64_t)key * p.k_pos + 8 * grp + 32 * c);
+            kr[hf * DC + c] = load16_nt(kb + (int64_t)key * p.k_pos + 8 * grp + 32 * c);
         }
 #pragma unroll
         for (int i = 0; i < VL; ++i) {
           const int r = (64 * i + lane) / CPR, pc = lane % CPR;
-          const int chunk = 2 * ((pc >> 1) ^ stream_swizzle<D>(r)) + (pc & 1);
-          const uint32_t key = min(base + (uint32_t)stream_slot_key(r), k1 - 1);
+          const int chunk = 2 * ((pc >> 1) ^ decode_v_swizzle<D>(r)) + (pc & 1);
+          const uint32_t key = min(base + (uint32_t)decode_slot_key(r), k1 - 1);
           load_lds16_nt(vb + (int64_t)key * p.v_pos + chunk * 8, vdst + i * 512);
         }
       }
     };
-    auto compute = [&](uint32_t ti, const uint4 *kr, const uint16_t *vst) __attribute__((always_inline)) {
+    // `finite` is a constant of the main loop: every value of the tile is.
+    auto compute = [&](uint32_t ti, const uint4 *kr, const uint16_t *vst, bool finite) __attribute__((always_inline)) {
       const uint32_t base = k0 + ti * KT;
       sf4_t s[2];  // s[hf][e]: head col, key 16 hf + 4 grp + e
 #pragma unroll
@@ -959,6 +942,15 @@ __global__ __launch_bounds__(kStreamWaves * 64, kStreamPerCu) void attn_decode_s
         m_run = m_new;
       }
       const float mc = m_run == -INFINITY ? 0.0f : m_run * c2 - kBias;
+      if (!finite) {
+        float w[2][4];
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w[hf][e] = exp2_raw(fmaf(s[hf][e], c2, -mc));
+        weigh_tile<D>(o, w, vst + wave * STAGE, v_lds_b + wave * STAGE, grp, col, (int)min(k1 - base, (uint32_t)KT));
+        return;
+      }
       uint32_t pw[4], pl[4];  // P as f16 pairs in the PV operand's key order (and its low terms)
       float ps = 0.0f;
 #pragma unroll
@@ -999,12 +991,12 @@ __global__ __launch_bounds__(kStreamWaves * 64, kStreamPerCu) void attn_decode_s
     while (ti < ntiles) {
       uint32_t nx = ti + WAVES;
       if (nx < ntiles) issue(nx, krb, v_lds_b);
-      compute(ti, kra, v_lds_a);
+      compute(ti, kra, v_lds_a, true);
       ti = nx;
       if (ti >= ntiles) break;
       nx = ti + WAVES;
       if (nx < ntiles) issue(nx, kra, v_lds_a);
-      compute(ti, krb, v_lds_b);
+      compute(ti, krb, v_lds_b, true);
       ti = nx;
     }
     l_run += __shfl_xor(l_run, 16, 64);
@@ -1012,37 +1004,22 @@ __global__ __launch_bounds__(kStreamWaves * 64, kStreamPerCu) void attn_decode_s
     if constexpr (SPLIT_P) {
       // An infinite or NaN value row times a zero weight (an empty low term, a
       // masked re-read key) is NaN in the products above. If any accumulator is
-      // not finite, the wave takes its tiles again on the vector units with
-      // whole f32 weights.
+      // not finite, the wave takes its tiles again, those that hold such a value
+      // on the vector units with whole f32 weights.
       float bad = 0.0f;
 #pragma unroll
       for (int dt = 0; dt < DB; ++dt) bad += (o[dt][0] + o[dt][1] + o[dt][2] + o[dt][3]) * 0.0f;
       if (__any(!(bad == 0.0f))) {
-        const float mc = m_run == -INFINITY ? 0.0f : m_run * c2 - kBias;
+        const float l_sum = l_run;
 #pragma unroll
         for (int dt = 0; dt < DB; ++dt) o[dt] = sf4_t{0.0f, 0.0f, 0.0f, 0.0f};
-        for (uint32_t t = wave; t < ntiles; t += WAVES)
-          for (uint32_t key = k0 + t * KT; key < min(k1, k0 + (t + 1) * KT); ++key) {
-            const uint16_t *kp = kb + (int64_t)key * p.k_pos, *vp = vb + (int64_t)key * p.v_pos;
-            float sc = 0.0f;
-#pragma unroll
-            for (int c = 0; c < DC; ++c) {
-              const uint4 kv = *reinterpret_cast<const uint4 *>(kp + 8 * grp + 32 * c);
-              const uint4 qv = __builtin_bit_cast(uint4, qop[c]);
-              sc = dot2(qv.x, kv.x, sc);
-              sc = dot2(qv.y, kv.y, sc);
-              sc = dot2(qv.z, kv.z, sc);
-              sc = dot2(qv.w, kv.w, sc);
-            }
-            sc += __shfl_xor(sc, 16, 64);
-            sc += __shfl_xor(sc, 32, 64);
-            const float wgt = exp2_raw(fmaf(sc, c2, -mc));
-#pragma unroll
-            for (int dt = 0; dt < DB; ++dt)
-#pragma unroll
-              for (int e = 0; e < 4; ++e)
-                o[dt][e] = fmaf(wgt, f16_to_f32(vp[16 * dt + 4 * grp + e]), o[dt][e]);
-          }
+#pragma unroll 1
+        for (uint32_t t = wave; t < ntiles; t += WAVES) {
+          issue(t, kra, v_lds_a);
+          __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+          compute(t, kra, v_lds_a, !any_not_finite<2 * STAGE>(v_lds_a + wave * STAGE, lane));
+        }
+        l_run = l_sum;
       }
     }
 

@@ -29,9 +29,10 @@ using namespace mi::dev;
 
 constexpr int BN = kPrefillBlockN;
 constexpr int BM = kPrefillBlockM;
-// Added to every probability's exponent: weights are at most 2^(kBias + 8) (the
-// lazy rescale), and a weight of 2^-16 of the largest still has 11 bits in its
-// low f16 term.
+// Added to every probability's exponent, so that the low f16 term of a weight of
+// 2^-8 of the largest still has its 11 bits above f16's smallest value (2^-24); a
+// smaller weight's pair is 2^-31 of the largest weight off at most. Weights are at
+// most 2^(kBias + 8) (the lazy rescale).
 constexpr float kBias = 6.0f;
 
 typedef float f4_t __attribute__((ext_vector_type(4)));
@@ -42,6 +43,7 @@ __global__ __launch_bounds__(256, 2) void attn_tiled_kernel(const PrefillParams 
   constexpr int DC = D / 16, DT = D / 32;
   __shared__ __attribute__((aligned(16))) uint16_t k_lds_a[BN * D], k_lds_b[BN * D];
   __shared__ __attribute__((aligned(16))) uint16_t v_lds_a[BN * D], v_lds_b[BN * D];
+  __shared__ uint32_t s_redo;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int n = lane & 31, h = lane >> 5;
   const uint32_t G = p.group;
@@ -112,6 +114,7 @@ __global__ __launch_bounds__(256, 2) void attn_tiled_kernel(const PrefillParams 
       qop[c] = row_ok ? as_h8(*reinterpret_cast<const uint4 *>(qrow + 16 * c + 8 * h))
                       : as_h8(make_uint4(0, 0, 0, 0));
   }
+  if (tid == 0) s_redo = 0;
   issue_tile(t_begin, k_lds_a, v_lds_a);
   if (t_begin + 1 < t_end) {
     issue_tile(t_begin + 1, k_lds_b, v_lds_b);
@@ -121,8 +124,8 @@ __global__ __launch_bounds__(256, 2) void attn_tiled_kernel(const PrefillParams 
     __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
   }
   // Bare barrier: a workgroup fence would wait for the second tile too. Each
-  // wave has waited for its own part of the first.
-  asm volatile("s_barrier" ::: "memory");
+  // wave has waited for its own part of the first, and for s_redo.
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
   float16_t o[DT];
 #pragma unroll
@@ -137,7 +140,8 @@ __global__ __launch_bounds__(256, 2) void attn_tiled_kernel(const PrefillParams 
   const int tr_off = tr_key * D + 4 * (tr_a & 1);
   const int tr_chunk = 2 * (tr_g & 1) + (tr_a >> 1);
 
-  auto compute = [&](uint32_t it, const uint16_t *k_lds, const uint16_t *v_lds) __attribute__((always_inline)) {
+  // `finite` (a constant of each call): P V on MFMA, which every value has to be for.
+  auto compute = [&](uint32_t it, const uint16_t *k_lds, const uint16_t *v_lds, bool finite) __attribute__((always_inline)) {
     const uint32_t j0 = it * BN;
     float16_t s[2];
 #pragma unroll
@@ -192,6 +196,37 @@ __global__ __launch_bounds__(256, 2) void attn_tiled_kernel(const PrefillParams 
         ps1 += s[mt][r + 1];
       }
     l_run += ps0 + ps1;
+    if (!finite) {
+      // P V on the vector units: the wave's weights go through LDS (the second
+      // stage, 32 keys at a time), and each lane adds the keys that its row sees
+      // to its d = 32 dt + 8 q + 4 h + e.
+      float *weights = reinterpret_cast<float *>((wave < 2 ? k_lds_b : v_lds_b) + (wave & 1) * 2048);
+      const int last = (int)max(min((int64_t)lim - (int64_t)j0, (int64_t)BN), (int64_t)-1);
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) weights[(8 * (r >> 2) + 4 * h + (r & 3)) * 32 + n] = s[mt][r];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma clang loop unroll_count(D == 64 ? 2 : 1)
+        for (int key = 0; key < 32; ++key) {
+          const float f = weights[key * 32 + n];
+          const uint16_t *row = v_lds + (32 * mt + key) * D + 4 * h;
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              uint2 v = *reinterpret_cast<const uint2 *>(row + ((4 * dt + q) ^ v_swizzle<D>(key)) * 8);
+              if (32 * mt + key > last) v = make_uint2(0, 0);
+              o[dt][4 * q] = fmaf(f, lo_f16(v.x), o[dt][4 * q]);
+              o[dt][4 * q + 1] = fmaf(f, hi_f16(v.x), o[dt][4 * q + 1]);
+              o[dt][4 * q + 2] = fmaf(f, lo_f16(v.y), o[dt][4 * q + 2]);
+              o[dt][4 * q + 3] = fmaf(f, hi_f16(v.y), o[dt][4 * q + 3]);
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      }
+      return;
+    }
     // O^T[d][row] += V^T[d][keys] P^T[keys][row], four 16-key chunks, P's low
     // terms first.
 #pragma unroll
@@ -219,56 +254,49 @@ __global__ __launch_bounds__(256, 2) void attn_tiled_kernel(const PrefillParams 
   // Tile t_begin + k lives in stage k & 1: after a tile its successor (issued a
   // tile ago) has landed, and past the barrier nobody reads this stage, which
   // takes the tile after that.
-  for (uint32_t it = t_begin; it < t_end; it += 2) {
-    if (busy) compute(it, k_lds_a, v_lds_a);
+  for (uint32_t it = t_begin;; it += 2) {
+    if (busy) compute(it, k_lds_a, v_lds_a, true);
+    if (it + 1 >= t_end) break;
     __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
     __syncthreads();
-    if (it + 1 >= t_end) break;
     if (it + 2 < t_end) issue_tile(it + 2, k_lds_a, v_lds_a);
-    if (busy) compute(it + 1, k_lds_b, v_lds_b);
+    if (busy) compute(it + 1, k_lds_b, v_lds_b, true);
+    if (it + 2 >= t_end) break;
     __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
     __syncthreads();
     if (it + 3 < t_end) issue_tile(it + 3, k_lds_b, v_lds_b);
   }
-
   // An infinite or NaN value row times a zero weight (a masked key, an empty low
-  // term) is NaN in the products above. If any accumulator is not finite, the
-  // wave takes its rows again on the vector units, visible keys only and with
-  // whole f32 weights.
-  {
-    float bad = 0.0f;
+  // term) is NaN in the products above: a wave with an accumulator that is not
+  // finite says so at the last tile's barrier.
+  float sum = 0.0f;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+  for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) bad = fmaf(o[dt][r], 0.0f, bad);
-    if (__any(!(bad == 0.0f))) {
-      const float mc = m_run == -INFINITY ? 0.0f : m_run * c2 - kBias;
+    for (int r = 0; r < 16; ++r) sum = fmaf(o[dt][r], 0.0f, sum);
+  const bool bad = __any(!(sum == 0.0f));
+  if (bad && lane == 0) s_redo = 1;
+  __syncthreads();
+  // Then the workgroup's tiles are loaded again, and the waves that have such an
+  // accumulator take them again on the vector units, visible keys only and with whole f32
+  // weights (MFMA for the tiles without such a value costs the main loop its
+  // registers: 16 spilled).
+  if (s_redo != 0) {
+    const float l_sum = l_run;
+    if (bad)
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[dt][r] = 0.0f;
-      for (uint32_t key = t_begin * BN; key < min(kmax, t_end * BN); ++key) {
-        const uint16_t *kp = kbase + (int64_t)key * p.k_pos, *vp = vbase + (int64_t)key * p.v_pos;
-        float sc = 0.0f;
-#pragma unroll
-        for (int c = 0; c < DC; ++c) {
-          const uint4 kv = *reinterpret_cast<const uint4 *>(kp + 16 * c + 8 * h);
-          const uint4 qv = __builtin_bit_cast(uint4, qop[c]);
-          sc = dot2(qv.x, kv.x, sc);
-          sc = dot2(qv.y, kv.y, sc);
-          sc = dot2(qv.z, kv.z, sc);
-          sc = dot2(qv.w, kv.w, sc);
-        }
-        sc += __shfl_xor(sc, 32, 64);
-        if (key > lim) continue;
-        const float w = exp2_raw(fmaf(sc, c2, -mc));
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            o[dt][r] = fmaf(w, f16_to_f32(vp[32 * dt + 8 * (r >> 2) + 4 * h + (r & 3)]), o[dt][r]);
-      }
+#pragma unroll 1
+    for (uint32_t it = t_begin; it < t_end; ++it) {
+      issue_tile(it, k_lds_a, v_lds_a);
+      __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+      __syncthreads();
+      if (bad) compute(it, k_lds_a, v_lds_a, false);
+      __syncthreads();
     }
+    l_run = l_sum;
   }
   const float l_total = l_run + __shfl_xor(l_run, 32, 64);
   if (n_tiles > per_split) {
