@@ -44,9 +44,11 @@ def run(ctx, q, k, v, lengths, hq, hkv, d, cap):
     (32, 8, 128, 1200, [1200] * 20),                        # past the pieces: equal segments
     (40, 8, 128, 500, [500, 33, 64, 0, 499]),               # groups of 5
     (34, 2, 128, 400, [400, 399]),                          # groups of 17: chunks of 9 and 8
-    (40, 8, 64, 1000, [1000, 33, 64, 0, 999]),
-    (16, 8, 64, 800, [(b * 97) % 801 for b in range(17)]),
+    (64, 8, 64, 1000, [1000, 33, 64, 0, 999]),
     (64, 8, 64, 3000, [3000, 2999, 1, 768] * 4),
+    (40, 8, 64, 800, [(b * 97) % 250 for b in range(60)] + [800]),  # groups of 5, pieces
+    (34, 2, 64, 800, [(b * 97) % 801 for b in range(70)]),          # chunks of 9 and 8
+    (8, 2, 64, 8192, [(b * 97) % 300 for b in range(90)]),          # groups of 4 by the capacity
 ])
 def test_batched_decode_work_split(ctx, hq, hkv, d, cap, lengths):
     B = len(lengths)
@@ -64,9 +66,46 @@ def test_batched_decode_work_split(ctx, hq, hkv, d, cap, lengths):
             assert (np.abs(f16(got[b:b + 1]).astype(np.float64) - ref["f32"]) <= bound).all()
 
 
+@pytest.mark.parametrize("hq,hkv,cap,B", [
+    (32, 8, 4096, 8),    # groups of 4, few sequences
+    (32, 8, 1024, 32),   # two rows splits of each unit
+    (32, 8, 1024, 70),   # more units than workgroups
+    (64, 8, 1024, 70),
+    (40, 8, 1024, 8),    # fewer than nine heads per CU
+    (16, 8, 1024, 20),
+    (8, 1, 4096, 8),     # one KV head
+    (64, 8, 700, 8),     # one rows split
+])
+def test_short_sequences_at_head_dim_64_stay_on_the_rows_kernel(ctx, hq, hkv, cap, B):
+    """Calls whose sequences may be short, where the rows kernel's one launch is the faster one."""
+    d, lengths = 64, [1 + (7 * b) % 60 for b in range(B)]
+    q, k, v = rand(1, (B, hq, d), 2.0), rand(2, (B, 64, hkv, d)), rand(3, (B, 64, hkv, d))
+    kt = ctx.empty((B, cap, hkv, d))
+    vt = ctx.empty((B, cap, hkv, d))
+    pad = np.zeros((B, cap - 64, hkv, d), np.uint16)
+    ctx.upload(kt, np.concatenate([k, pad], 1))
+    ctx.upload(vt, np.concatenate([v, pad], 1))
+    qt, lt = ctx.tensor(q), ctx.tensor(np.asarray(lengths, np.uint32), mi_attn.U32)
+    ctx.take_kernel_profiles()
+    ctx.set_kernel_profiling(True)
+    try:
+        batch = ctx.begin_batch()
+        out = batch.attention_decode_batched(qt, kt, vt, lt, mi_attn.AttentionConfig(hq, hkv, d, True, 0))
+        batch.finish()
+        names = [name for name, _ in ctx.take_kernel_profiles()]
+    finally:
+        ctx.set_kernel_profiling(False)
+    assert names == ["attn_rows_batched"], names
+    got = ctx.download(out)
+    for b in range(0, B, 5):
+        n = lengths[b]
+        ref = oracle_attention(q[b:b + 1], k[b, :n], v[b, :n], hq=hq, hkv=hkv, d=d, off=n - 1)
+        assert_parity(got[b:b + 1], ref, label=f"seq {b} len {n}")
+
+
 def test_batched_decode_with_infinite_values_at_head_dim_64(ctx):
     """An infinite value gives the infinity that the weighted sum gives, in its own column only."""
-    hq, hkv, d, cap, lengths = 32, 8, 64, 800, [800, 37, 300, 65] * 4
+    hq, hkv, d, cap, lengths = 64, 8, 64, 800, [800, 37, 300, 65] * 4
     q, k, v = rand(4, (16, hq, d)), rand(5, (16, cap, hkv, d)), rand(6, (16, cap, hkv, d))
     for b, n in enumerate(lengths):
         v[b, n - 1, b % hkv, b] = np.float16(np.inf if b % 2 else -np.inf).view(np.uint16)
