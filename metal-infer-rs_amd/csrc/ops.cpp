@@ -815,34 +815,33 @@ mi_status decode_batched(mi_batch *batch, const mi_tensor *q, const mi_tensor *k
       kv_units * ceil_div(p.G, kernels::kDecodeRows) <= kernels::stream_workgroups(cus) &&
       (p.G == 8 || kv_units * p.G >= 9 * cus ||
        (p.G == 4 && kv_units * ceil_div(p.L, kRowsBatchedBlock) >= 6 * cus));
-  bool stream = block_keys == 0 && (uint64_t)B <= kernels::kStreamMaxBatch &&
-                pos_stride_fits_u32(k->stride[1], v->stride[1], 32) && (p.D == 128 || stream64);
-  uint64_t bytes = 0;
-  uint32_t unit_slots = 0;
+  const bool stream = block_keys == 0 && (uint64_t)B <= kernels::kStreamMaxBatch &&
+                      pos_stride_fits_u32(k->stride[1], v->stride[1], 32) && (p.D == 128 || stream64);
   if (stream) {
+    rp.group = p.G, rp.stream_workgroups = kernels::stream_workgroups(batch->ctx->compute_units);
+    auto partial_bytes = [&](uint32_t chunks, uint32_t slots) -> uint64_t {
+      return kernels::stream_partial_floats(kv_units * chunks, rp.stream_workgroups, ceil_div(p.G, chunks),
+                                            slots, p.D) *
+             sizeof(float);
+    };
+    // The fewest head chunks, each of which reads K/V: unless their partials pass
+    // the no-allocation buffer where those of the largest power-of-two chunks that
+    // divide the group fit it (more chunks, but smaller overflow slots). The choice
+    // moves the pieces' boundaries and so the rounding, and is the same with and
+    // without that buffer.
+    rp.head_chunks = std::max(1u, ceil_div(p.G, kernels::kDecodeRows));
+    if (partial_bytes(rp.head_chunks, 0) > kNoAllocScratchBytes) {
+      uint32_t chunks = rp.head_chunks;
+      while (p.G % chunks != 0 || !pow2(p.G / chunks)) ++chunks;
+      if (partial_bytes(chunks, 0) <= kNoAllocScratchBytes) rp.head_chunks = chunks;
+    }
+    rp.rows = ceil_div(p.G, rp.head_chunks);
     // Fixed slots per unit, so that the merge loads a unit's pieces with its
     // descriptor; a fixed buffer too small for them takes the compact layout
-    // (every piece in an overflow slot, same merge order and results), and then
-    // the largest power-of-two chunks that divide the group, whose overflow
-    // slots are the smallest. At head_dim 64 the rows kernel, whose partials
-    // grow with the capacity instead of the sequences, is left after that.
-    rp.group = p.G, rp.stream_workgroups = kernels::stream_workgroups(batch->ctx->compute_units);
-    for (int attempt = 0; attempt < 3; ++attempt) {
-      rp.head_chunks = std::max(1u, ceil_div(p.G, kernels::kDecodeRows));
-      if (attempt == 2 && p.G != 0)
-        for (rp.head_chunks = 1; p.G % rp.head_chunks != 0 || !pow2(p.G / rp.head_chunks) ||
-                                 p.G / rp.head_chunks > kernels::kDecodeRows;)
-          ++rp.head_chunks;
-      rp.rows = ceil_div(p.G, rp.head_chunks);
-      unit_slots = attempt == 0 ? kernels::kStreamUnitSlots : 0;
-      bytes = kernels::stream_partial_floats((uint64_t)B * p.Hkv * rp.head_chunks, rp.stream_workgroups,
-                                             rp.rows, unit_slots, p.D) *
-              sizeof(float);
-      if (src.fixed == nullptr || bytes <= src.limit) break;
-    }
-    if (p.D == 64 && src.fixed != nullptr && bytes > src.limit) stream = false;
-  }
-  if (stream) {
+    // (every piece in an overflow slot, same merge order and results).
+    uint32_t unit_slots = kernels::kStreamUnitSlots;
+    if (src.fixed != nullptr && partial_bytes(rp.head_chunks, unit_slots) > src.limit) unit_slots = 0;
+    const uint64_t bytes = partial_bytes(rp.head_chunks, unit_slots);
     rp.stream_unit_slots = unit_slots;
     void *scratch = nullptr;
     if ((st = scratch_take(batch, src, bytes, &scratch)) != MI_OK) return st;

@@ -66,6 +66,23 @@ def test_batched_decode_work_split(ctx, hq, hkv, d, cap, lengths):
             assert (np.abs(f16(got[b:b + 1]).astype(np.float64) - ref["f32"]) <= bound).all()
 
 
+@pytest.mark.parametrize("B,hq,hkv,cap", [
+    (900, 34, 1, 40),   # compact, with chunks that divide the group: 17 of 2 heads
+    (700, 34, 1, 40),   # compact: three chunks of 12, 12 and 10
+    (200, 34, 1, 40),   # fixed slots
+])
+def test_batched_decode_of_wide_groups_in_the_fixed_buffer(ctx, B, hq, hkv, cap):
+    """Near the fixed buffer's size the call without allocations still gives the other call's bits,
+    so the head chunks, which move the pieces' boundaries, are the same in both."""
+    lengths = [1 + (11 * b) % cap for b in range(B)]
+    q, k, v = rand(1, (B, hq, 128), 2.0), rand(2, (B, cap, hkv, 128)), rand(3, (B, cap, hkv, 128))
+    got, _ = run(ctx, q, k, v, lengths, hq, hkv, 128, cap)  # compares the two calls
+    for b in range(0, B, 97):
+        n = lengths[b]
+        ref = oracle_attention(q[b:b + 1], k[b, :n], v[b, :n], hq=hq, hkv=hkv, d=128, off=n - 1)
+        assert_parity(got[b:b + 1], ref, label=f"seq {b} len {n}")
+
+
 @pytest.mark.parametrize("hq,hkv,cap,B", [
     (32, 8, 4096, 8),    # groups of 4, few sequences
     (32, 8, 1024, 32),   # two rows splits of each unit
