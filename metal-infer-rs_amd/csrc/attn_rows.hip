@@ -1099,10 +1099,16 @@ __global__ __launch_bounds__(kStreamWaves * 64, kStreamPerCu) void attn_decode_s
 // against 107.7-107.9 us per call). One thread per output element (GC x 128,
 // at least 256, at most 1024), so the slots load in one pass (c4, GQA 4:
 // 105.7 against 106.0 us with 256 threads and two passes, bit-identical).
-template <int D>
+// FEW (launches of at most 128 units, which leave CUs idle): more than 1024 elements
+// (groups past 8 heads at D = 128) take two workgroups of a unit, and more than 24
+// pieces 16 per pass; a pass is one dependent round trip. Four sequences of 1024 to
+// 8192 keys, 24/2 heads 31.0 -> 24.1 us; one of 6189, 14/2 20.1 -> 19.2. Past that
+// the second workgroup and the registers of 16 pieces cost more than they give
+// (128 sequences of 300 keys, 128/8 heads 42.3 -> 47.6).
+template <int D, bool FEW>
 __global__ __launch_bounds__(1024) void attn_stream_merge_kernel(const RowsParams p) {
   constexpr int ROW = D + 2;
-  constexpr int C = kStreamUnitSlots;  // pieces per pass
+  constexpr int C = kStreamUnitSlots, CO = FEW ? 16 : C;  // pieces per pass: own slots, overflow
   const uint32_t S = p.stream_unit_slots;
   const uint32_t upb = p.kv_heads * p.head_chunks;
   const uint32_t unit = blockIdx.x, b = unit / upb, j = unit % upb;
@@ -1115,12 +1121,12 @@ __global__ __launch_bounds__(1024) void attn_stream_merge_kernel(const RowsParam
   const uint32_t kvh = j / p.head_chunks, hc = j % p.head_chunks;
   const uint32_t GC = min(p.rows, p.group - hc * p.rows);  // heads of this chunk
   uint16_t *out = p.out + (int64_t)b * p.o_seq + (int64_t)(kvh * p.group + hc * p.rows) * p.o_head;
-  for (uint32_t idx = threadIdx.x; idx < GC * D; idx += blockDim.x) {
+  for (uint32_t idx = blockIdx.y * blockDim.x + threadIdx.x; idx < GC * D; idx += gridDim.y * blockDim.x) {
     const int g = idx / D, d = idx % D;
     // The unit's own slots, issued before the descriptor is known (in
     // bounds whatever they hold). The compact layout (S = 0) has none: every
     // piece is loaded after the descriptor below.
-    float m[C], l[C], a[C];
+    float m[CO], l[CO], a[CO];
     if (S != 0) {
 #pragma unroll
       for (int i = 0; i < C; ++i) {
@@ -1133,36 +1139,45 @@ __global__ __launch_bounds__(1024) void attn_stream_merge_kernel(const RowsParam
     // Zero keys: NaN, written by the stream kernel (the descriptor is stale).
     const uint32_t pieces = desc >> 16;
     if (len_b == 0 || pieces <= 1) return;
-    const float *base = pieces <= S ? own : overflow + (size_t)((desc & 0xffff) + unit) * p.rows * ROW;
+    const float *base = overflow + (size_t)((desc & 0xffff) + unit) * p.rows * ROW;
     float M = -INFINITY, Ls = 0.0f, As = 0.0f;
-    for (uint32_t s0 = 0; s0 < pieces; s0 += C) {
-      if (pieces > S) {
+    // Folds N loaded pieces, `left` of them the unit's (slots past its last piece
+    // hold other data).
+    auto fold = [&](auto n_tag, uint32_t left) __attribute__((always_inline)) {
+      constexpr int N = decltype(n_tag)::value;
+      bool use[N];
 #pragma unroll
-        for (int i = 0; i < C; ++i) {
-          const float *ps = base + (size_t)(min(s0 + i, pieces - 1) * p.rows + g) * ROW;
-          m[i] = ps[0];
-          l[i] = ps[1];
-          a[i] = ps[2 + d];
-        }
-      }
-      // Slots past the last piece hold other data: they take no part.
-      bool use[C];
-#pragma unroll
-      for (int i = 0; i < C; ++i) use[i] = s0 + i < pieces && m[i] != -INFINITY;
+      for (int i = 0; i < N; ++i) use[i] = (uint32_t)i < left && m[i] != -INFINITY;
       float cm = M;
 #pragma unroll
-      for (int i = 0; i < C; ++i) cm = use[i] ? fmaxf(cm, m[i]) : cm;
+      for (int i = 0; i < N; ++i) cm = use[i] ? fmaxf(cm, m[i]) : cm;
       const float r = M == -INFINITY ? 0.0f : exp2_raw(M - cm);
       Ls *= r;
       As *= r;
 #pragma unroll
-      for (int i = 0; i < C; ++i) {
+      for (int i = 0; i < N; ++i) {
         const float f = use[i] ? exp2_raw(m[i] - cm) : 0.0f;
         Ls = use[i] ? fmaf(l[i], f, Ls) : Ls;
         As = use[i] ? fmaf(a[i], f, As) : As;
       }
       M = cm;
-    }
+    };
+    auto load_fold = [&](auto n_tag, uint32_t s0) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < decltype(n_tag)::value; ++i) {
+        const float *ps = base + (size_t)(min(s0 + i, pieces - 1) * p.rows + g) * ROW;
+        m[i] = ps[0];
+        l[i] = ps[1];
+        a[i] = ps[2 + d];
+      }
+      fold(n_tag, pieces - s0);
+    };
+    if (pieces <= S)
+      fold(std::integral_constant<int, C>{}, pieces);
+    else if (!FEW || pieces <= 3 * C)
+      for (uint32_t s0 = 0; s0 < pieces; s0 += C) load_fold(std::integral_constant<int, C>{}, s0);
+    else
+      for (uint32_t s0 = 0; s0 < pieces; s0 += CO) load_fold(std::integral_constant<int, CO>{}, s0);
     out[g * p.o_head + d] = f32_to_f16(As / Ls);
   }
 }
@@ -1253,8 +1268,11 @@ hipError_t launch_stream_d(const RowsParams &p, RowsPhase phase, const Launch &l
   if (phase == RowsPhase::Split)
     return dispatch(attn_decode_stream_kernel<D>, dim3(p.stream_workgroups), dim3(kStreamWaves * 64), 0, l, p);
   const uint32_t units = p.batch * p.kv_heads * p.head_chunks, outs = p.rows * D;
-  return dispatch(attn_stream_merge_kernel<D>, dim3(units), dim3(outs > 1024 ? 1024 : outs > 256 ? outs : 256),
-                  0, l, p);
+  const uint32_t blocks = units > 128 ? 1 : (outs + 1023) / 1024;
+  const uint32_t threads = ((outs + blocks - 1) / blocks + 63) / 64 * 64;
+  const dim3 grid(units, blocks), block(threads > 1024 ? 1024 : threads > 256 ? threads : 256);
+  if (units > 128) return dispatch(attn_stream_merge_kernel<D, false>, grid, block, 0, l, p);
+  return dispatch(attn_stream_merge_kernel<D, true>, grid, block, 0, l, p);
 }
 }  // namespace
 

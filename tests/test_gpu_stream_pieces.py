@@ -44,6 +44,7 @@ def run(ctx, q, k, v, lengths, hq, hkv, d, cap):
     (32, 8, 128, 1200, [1200] * 20),                        # past the pieces: equal segments
     (40, 8, 128, 500, [500, 33, 64, 0, 499]),               # groups of 5
     (34, 2, 128, 400, [400, 399]),                          # groups of 17: chunks of 9 and 8
+    (24, 2, 128, 4000, [4000, 3073, 37]),                   # 32 pieces of 12 heads: two merge workgroups
     (64, 8, 64, 1000, [1000, 33, 64, 0, 999]),
     (64, 8, 64, 3000, [3000, 2999, 1, 768] * 4),
     (40, 8, 64, 800, [(b * 97) % 250 for b in range(60)] + [800]),  # groups of 5, pieces
