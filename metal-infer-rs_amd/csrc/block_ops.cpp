@@ -271,7 +271,8 @@ mi_status mi_matmul(mi_batch *batch, const mi_tensor *input, const mi_tensor *we
   if (kernels::skinny_gemm_supported(p, cus))
     return launch(batch, "skinny_gemm",
                   [&](const kernels::Launch &l) { return kernels::launch_skinny_gemm(p, cus, l); });
-  // More rows, as long as one output tile per CU covers them.
+  // More rows, where one output tile per CU covers them and measured faster than
+  // the library.
   if (kernels::gemm_tile_supported(p, cus))
     return launch(batch, "gemm_tile",
                   [&](const kernels::Launch &l) { return kernels::launch_gemm_tile(p, cus, l); });

@@ -3,14 +3,15 @@
 // tile per CU.
 //
 // What bounds it: at these sizes one round of tiles is the whole launch, so the
-// time is one workgroup's walk along k, its loads per step at a CU's L2 rate plus
-// whatever of the load latency is not covered. So the k steps run through a ring
+// time is one workgroup's walk along k, its loads per step: 45 to 60 bytes per ns
+// and CU in the traces, with two or more stages in flight. Whether that is the L2's
+// rate or its latency under load is not told apart. So the k steps run through a ring
 // of LDS stages filled by direct loads (96 to 147 KB), and the tile is the one
 // with the least rows of x and w that still fits all tiles on the chip at once.
 // Measured on MI355X (graph replays over rotated weights, hipBLASLt -> this):
-// [128, 2048] x [1024, 2048]^T 8.3 -> 6.4 us, 48 x [1024, 1024] 8.1 -> 4.7, 100 x
-// [2048, 2048] 11.1 -> 7.6, 1100 x [2048, 2048] 22.9 -> 19.1, 2048 x [1024, 2048]
-// 16.0 -> 15.0, 256 x [5120, 8192] 73 -> 49.
+// [128, 2048] x [1024, 2048]^T 8.4 -> 6.4 us, 48 x [1024, 1024] 8.1 -> 4.7, 100 x
+// [2048, 2048] 8.4 -> 6.4, 1100 x [2048, 2048] 18.6 -> 16.8, 2048 x [1024, 2048]
+// 14.7 -> 13.4, 256 x [5120, 8192] 72 -> 49.
 //  - 8 waves: two groups of 2 x 2. Each group multiplies half of every step's
 //    keys for the whole tile (two waves per SIMD hide each other's LDS reads at
 //    the LDS traffic of 2 x 2), and the second group's sums are added through LDS.
@@ -176,46 +177,89 @@ __global__ __launch_bounds__(512, 2) void gemm_tile_kernel(const MatvecParams p,
     }
 }
 
+template <int BM, int BN>
+struct TileGrid {
+  uint64_t row_tiles, col_tiles, tiles;
+  TileGrid(const MatvecParams &p)
+      : row_tiles((p.m + BM - 1ull) / BM), col_tiles((p.n + BN - 1ull) / BN), tiles(row_tiles * col_tiles) {}
+  // Real rows of x in the row tiles, and real elements in all tiles, in percent.
+  uint64_t row_fill(const MatvecParams &p) const { return 100ull * p.m / (row_tiles * BM); }
+  uint64_t fill(const MatvecParams &p) const { return row_fill(p) * p.n / (col_tiles * BN); }
+};
+
 template <int BM, int BN, int BK, int S>
-bool run_tile(const MatvecParams &p, uint32_t compute_units, const Launch *l, hipError_t *err) {
-  const uint64_t row_tiles = (p.m + BM - 1ull) / BM;
-  const uint64_t col_tiles = (p.n + BN - 1ull) / BN, tiles = row_tiles * col_tiles;
-  if (tiles > compute_units) return false;
-  if (l != nullptr)
-    *err = dispatch(gemm_tile_kernel<BM, BN, BK, S>, dim3((uint32_t)(tiles + kXcds - 1) / kXcds * kXcds),
-                    dim3(512), 0, *l, p, (uint32_t)row_tiles, (uint32_t)col_tiles);
-  return true;
+hipError_t run_tile(const MatvecParams &p, const Launch &l) {
+  const TileGrid<BM, BN> g(p);
+  return dispatch(gemm_tile_kernel<BM, BN, BK, S>, dim3((uint32_t)(g.tiles + kXcds - 1) / kXcds * kXcds), dim3(512),
+                  0, l, p, (uint32_t)g.row_tiles, (uint32_t)g.col_tiles);
 }
 
-// Launches (with `l`) the tile with the least rows of x and w together whose tiles
-// fit the chip at once; false where the library is the faster one: if none fits
-// (4096 x [5120, 8192] runs at 1.2 PFLOP/s there), and for long rows of w either
-// with the narrow tiles (48 x [5120, 8192] 28.2 us there, 30.1 here) or with the
-// largest (400 x [5120, 8192] 63.1 / 67.0; at k = 5120 43.5 / 42.4).
-bool pick_tile(const MatvecParams &p, uint32_t compute_units, const Launch *l, hipError_t *err) {
-  if (run_tile<32, 32, 128, 6>(p, compute_units, p.k <= 4096 ? l : nullptr, err)) return p.k <= 4096;
-  if (run_tile<64, 32, 128, 6>(p, compute_units, p.k <= 4096 ? l : nullptr, err)) return p.k <= 4096;
-  return run_tile<64, 64, 128, 4>(p, compute_units, l, err) ||
-         run_tile<64, 96, 128, 3>(p, compute_units, l, err) ||
-         run_tile<128, 64, 128, 3>(p, compute_units, l, err) ||
-         (p.k <= 5120 && run_tile<192, 64, 64, 4>(p, compute_units, l, err));
+// The tile with the least rows of x and w together whose tiles fit the chip at once;
+// None where the library measured faster (m = 33 to 3072 in 70 steps for 21 shapes of
+// w from 1024 x 1024 to 8192 x 8192 and 4096 x 11008, and 16 others that drew no line;
+// library / this in us). A tile's
+// time goes by the real rows in it, the library's by its own larger tiles, so the
+// lines are k, the share of the CUs and the share of real rows: where this says a
+// tile, the worst is 5% (208 x [5120, 5120] 29.4 / 30.9; 224 of them 46.2 / 32.2).
+//  - If none fits: 4096 x [5120, 8192] runs at 1.2 PFLOP/s in the library.
+//  - 32 x 32: k up to 2048. 48 x [1536, 3072] 7.6 / 8.1, 64 x [1024, 4096] 8.3 / 9.8.
+//  - 64 x 32: k up to 3584, or past 64 rows (64 x [5120, 4096] 17.6 / 18.4, 128 x [4096,
+//    4096] 24.4 / 17.2).
+//  - 64 x 64: from k = 4096 more than one row tile takes 60% of the CUs, up to 95 rows
+//    70% (160 x [2816, 5632] 22.0 / 25.4; 90 x [5120, 5120] 22.0 / 25.3, [5120, 8192]
+//    29.5 / 33.6; 96 of them 27.9 / 25.9).
+//  - 64 x 96: k up to 2048, or 4096 for narrow w, two row tiles or less, or padding: 512 x
+//    [2560, 4096] 23.7 / 25.2, 400 of them 24.8 / 23.1; 320 x [4096, 11008] 62 / 66, 700 x
+//    [1536, 8960] 44.6 / 50.3.
+//  - 128 x 64: past k = 1024 only on more than 3/4 of the CUs (384 x [4096, 4096] 24.9 /
+//    28.2, 400 of them 25.7 / 24.9), past 4096 also not half empty (144 x [8192, 8192]
+//    47.1 / 50.6).
+//  - 192 x 64: three row tiles or more (300 x [6144, 2048] 17.9 / 19.2) and k up to 2048,
+//    else to 5120 for wide w on nearly all CUs with some padding (768 x [3072, 3072]
+//    27.4 / 30.2, 832 of them 27.4 / 25.9; 576 x [5120, 5120] 45.4 / 49.0).
+enum class Tile { None, T32x32, T64x32, T64x64, T64x96, T128x64, T192x64 };
+
+Tile pick_tile(const MatvecParams &p, uint64_t cus) {
+  if (TileGrid<32, 32>(p).tiles <= cus) return p.k <= 2048 ? Tile::T32x32 : Tile::None;
+  if (TileGrid<64, 32>(p).tiles <= cus) return p.k <= 3584 || (p.k <= 4096 && p.m > 64) ? Tile::T64x32 : Tile::None;
+  if (const TileGrid<64, 64> g(p); g.tiles <= cus)
+    return p.k < 4096 || p.m <= 64 || 10 * g.tiles >= (p.m < 96 ? 7 : 6) * cus ? Tile::T64x64 : Tile::None;
+  if (const TileGrid<64, 96> g(p); g.tiles <= cus)
+    return p.k <= 2048 || (p.k <= 4096 && p.n <= 1536) || p.m <= 128 || (p.k <= 8192 && (p.m <= 256 || g.fill(p) <= 92))
+               ? Tile::T64x96
+               : Tile::None;
+  if (const TileGrid<128, 64> g(p); g.tiles <= cus)
+    return p.k <= 1024 || (4 * g.tiles > 3 * cus && (p.k < 4096 || g.row_fill(p) >= 72)) ? Tile::T128x64
+                                                                                        : Tile::None;
+  if (const TileGrid<192, 64> g(p); g.tiles <= cus)
+    return p.m > 384 && (p.k <= 2048 || (p.k <= 5120 && p.n >= 3072 && 100 * g.tiles >= 93 * cus &&
+                                         g.row_fill(p) <= 92))
+               ? Tile::T192x64
+               : Tile::None;
+  return Tile::None;
 }
 
 }  // namespace
 
 bool gemm_tile_supported(const MatvecParams &p, uint32_t compute_units) {
   auto aligned = [](const void *ptr, uintptr_t to) { return reinterpret_cast<uintptr_t>(ptr) % to == 0; };
-  hipError_t err = hipSuccess;
   return p.m > kSkinnyMaxRows && p.n > 0 && p.n % 4 == 0 && p.k > 0 && p.k % 128 == 0 &&
          p.x_row % 8 == 0 && p.w_row % 8 == 0 && p.o_row % 4 == 0 && aligned(p.x, 16) &&
-         aligned(p.w, 16) && aligned(p.out, 8) && pick_tile(p, compute_units, nullptr, &err);
+         aligned(p.w, 16) && aligned(p.out, 8) && pick_tile(p, compute_units) != Tile::None;
 }
 
 hipError_t launch_gemm_tile(const MatvecParams &p, uint32_t compute_units, const Launch &l) {
   if (!gemm_tile_supported(p, compute_units)) return hipErrorInvalidValue;
-  hipError_t err = hipErrorInvalidValue;
-  pick_tile(p, compute_units, &l, &err);
-  return err;
+  switch (pick_tile(p, compute_units)) {
+    case Tile::T32x32: return run_tile<32, 32, 128, 6>(p, l);
+    case Tile::T64x32: return run_tile<64, 32, 128, 6>(p, l);
+    case Tile::T64x64: return run_tile<64, 64, 128, 4>(p, l);
+    case Tile::T64x96: return run_tile<64, 96, 128, 3>(p, l);
+    case Tile::T128x64: return run_tile<128, 64, 128, 3>(p, l);
+    case Tile::T192x64: return run_tile<192, 64, 64, 4>(p, l);
+    case Tile::None: break;
+  }
+  return hipErrorInvalidValue;
 }
 
 }  // namespace kernels

@@ -205,7 +205,15 @@ def test_matmul_skinny_views(ctx, pad, offset):
     (1537, 1020, 512, 0, "gemm_tile"),   # 128 x 64, 13 row tiles: a band of 8 and one of 5
     (1101, 2048, 128, 0, "gemm_tile"),   # 192 x 64, two steps
     (1101, 2044, 576, 0, "gemm"),        # k no multiple of 128: library
-    (40, 5120, 5120, 0, "gemm"),         # narrow tiles, long rows: library
+    # Calls that the library does faster, by the tile that fits.
+    (40, 5120, 5120, 0, "gemm"),
+    (64, 1024, 4096, 0, "gemm"),         # 32 x 32, long rows
+    (70, 5120, 5120, 0, "gemm"),         # 64 x 64, second row tile nearly empty on few CUs
+    (96, 5120, 5120, 0, "gemm_tile"),
+    (512, 2560, 4096, 0, "gemm"),        # 64 x 96, no padding
+    (384, 4096, 4096, 0, "gemm"),        # 128 x 64 on 3/4 of the CUs
+    (768, 3072, 3072, 0, "gemm"),        # 192 x 64 on 3/4 of the CUs
+    (832, 3072, 3072, 0, "gemm_tile"),
 ])
 def test_matmul_tiled_rows(ctx, m, n, k, pad, kernel):
     """More than 32 rows: one output tile per CU, at each tile's remainders, and
