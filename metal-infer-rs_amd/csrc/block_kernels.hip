@@ -639,13 +639,21 @@ hipError_t launch_skinny_gemm(const MatvecParams &p, uint32_t compute_units, con
   return dispatch(skinny_gemm_kernel<2>, dim3(p.n / 16), dim3(256), 0, l, p);
 }
 
-bool stream_matmul_supported(const MatvecParams &p) {
+// Two and three rows of many features stay on the matvec where k is short: a
+// workgroup's eight waves take a 256-key chunk each, so below 2048 keys some idle,
+// and past 16 features per CU the launch has more than one round of such workgroups
+// (MI355X, graph replays over rotated weights, matvec / this in us: 2 x [5120, 256]
+// 3.4 / 3.8, [20000, 1024] 11.9 / 13.3, [32000, 512] 11.4 / 16.1, [5120, 2048] 6.4 / 6.8,
+// but [4096, 256] 3.1 / 2.8, [5120, 3072] 8.8 / 8.3; 3 x [32000, 512] 14.0 / 16.5, [32000,
+// 1280] 24.8 / 22.6; 4 rows win everywhere).
+bool stream_matmul_supported(const MatvecParams &p, uint32_t compute_units) {
+  if (p.n > 16ull * compute_units && p.k <= (p.m == 2 ? 2048u : p.m == 3 ? 1024u : 0u)) return false;
   return p.m > 1 && p.m <= kMatvecRows && p.n > 0 && p.k > 0 && p.k % kStreamMatmulChunk == 0 &&
          p.x_row % 8 == 0 && p.w_row % 8 == 0 && aligned16(p.x) && aligned16(p.w);
 }
 
 hipError_t launch_stream_matmul(const MatvecParams &p, uint32_t compute_units, const Launch &l) {
-  if (!stream_matmul_supported(p)) return hipErrorInvalidValue;
+  if (!stream_matmul_supported(p, compute_units)) return hipErrorInvalidValue;
   // The most features per workgroup that still give every CU one; past 16 per
   // CU, 8 with two workgroups per CU (8 x [5120, 8192]: 21.7 against 24.7 us).
   auto run = [&](auto feat_tag) {

@@ -260,14 +260,15 @@ mi_status mi_matmul(mi_batch *batch, const mi_tensor *input, const mi_tensor *we
   p.x = static_cast<const uint16_t *>(input->data), p.x_row = ldx;
   p.w = static_cast<const uint16_t *>(weight->data), p.w_row = ldw;
   p.out = static_cast<uint16_t *>(out->data), p.o_row = ldo;
-  // 9 to 32 rows (the batched-decode o_proj): the skinny GEMM where the
-  // grid fits the device; it measured 9.9 us against hipBLASLt's 12.1 us for
-  // [32, 4096] x [4096, 4096]^T.
+  // 2 to 8 rows: MFMA on the streamed weight.
   const uint32_t cus = batch->ctx->compute_units;
-  if (kernels::stream_matmul_supported(p))
+  if (kernels::stream_matmul_supported(p, cus))
     return launch(batch, "stream_matmul", [&](const kernels::Launch &l) {
       return kernels::launch_stream_matmul(p, cus, l);
     });
+  // 9 to 32 rows (the batched-decode o_proj): the skinny GEMM where the
+  // grid fits the device; it measured 9.9 us against hipBLASLt's 12.1 us for
+  // [32, 4096] x [4096, 4096]^T.
   if (kernels::skinny_gemm_supported(p, cus))
     return launch(batch, "skinny_gemm",
                   [&](const kernels::Launch &l) { return kernels::launch_skinny_gemm(p, cus, l); });

@@ -273,10 +273,10 @@ struct MatvecParams {
   uint32_t m, n, k;
 };
 constexpr uint32_t kMatvecRows = 8;
-// Two to kMatvecRows rows on MFMA: k % kStreamMatmulChunk == 0 and x, w rows
-// 16-byte aligned.
+// Two to kMatvecRows rows on MFMA: k % kStreamMatmulChunk == 0, x and w rows
+// 16-byte aligned, and not where the matvec is the faster one.
 constexpr uint32_t kStreamMatmulChunk = 256;
-bool stream_matmul_supported(const MatvecParams &p);
+bool stream_matmul_supported(const MatvecParams &p, uint32_t compute_units);
 hipError_t launch_stream_matmul(const MatvecParams &p, uint32_t compute_units, const Launch &l);
 // Skinny GEMM for kMatvecRows < m <= kSkinnyMaxRows, bound by streaming the
 // weight: one workgroup per 16 output features. Requires n % 16 == 0 with

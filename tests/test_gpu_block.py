@@ -194,6 +194,24 @@ def test_matmul_skinny_views(ctx, pad, offset):
     check_matmul(ctx.download(out), rows, w, f"view pad={pad} offset={offset}")
 
 
+@pytest.mark.parametrize("m,n,k,kernel", [
+    (2, 4096, 256, "stream_matmul"),   # 16 features per CU: one round
+    (2, 4100, 256, "matvec"),
+    (2, 4100, 2048, "matvec"),
+    (2, 4100, 2304, "stream_matmul"),  # a chunk of k for every wave, and one more
+    (3, 4100, 1024, "matvec"),
+    (3, 4100, 1280, "stream_matmul"),
+    (4, 4100, 256, "stream_matmul"),
+])
+def test_matmul_few_rows_of_many_features(ctx, m, n, k, kernel):
+    """Two and three rows: the matvec where the MFMA kernel's waves would idle (on 256 CUs)."""
+    x = rand(700 + m, (m, k))
+    w = rand(800 + n, (n, k), scale=k ** -0.5)
+    names, got = matmul_kernels(ctx, x, w)
+    assert names == [kernel], names
+    check_matmul(got, x, w, f"{m}x{n}x{k}")
+
+
 @pytest.mark.parametrize("m,n,k,pad,kernel", [
     (33, 4, 128, 0, "gemm_tile"),        # one step, one tile with four features
     (64, 100, 256, 8, "gemm_tile"),      # 32 x 32, fewer steps than stages, padded rows
