@@ -285,10 +285,12 @@ mi_status mi_attention_plan(const mi_context *ctx, const mi_tensor *q,
  * (values above C are clamped to C; a sequence of length 0 gets NaN, the
  * reference's 0/0); causal over each sequence (query at position
  * lengths[b] - 1). out [B, Hq, D]. config->query_offset is ignored.
- * block_keys = 0 picks the default: at head_dim 128, and mostly at 64, with
- * B <= 1024 an MFMA kernel whose workgroups share all sequences' keys equally
- * (stream-K; few keys: one piece of a unit per workgroup), otherwise the rows
- * kernel over a flat (sequence, KV head, split) grid.
+ * block_keys = 0 picks the default: at head_dim 128 with B <= 1024 an MFMA
+ * kernel whose workgroups share all sequences' keys equally (stream-K; few
+ * keys: one piece of a unit per workgroup), and at 64 too where short
+ * sequences would not make it the slower one (groups of 8, or many heads, and
+ * at most 2 units per CU); otherwise the rows kernel over a flat (sequence,
+ * KV head, split) grid.
  * block_keys > 0 runs the rows kernel with splits of that many keys. */
 mi_status mi_attention_decode_batched(mi_batch *batch, const mi_tensor *q,
                                       const mi_tensor *k, const mi_tensor *v,
@@ -420,8 +422,9 @@ mi_status mi_rope(mi_batch *batch, const mi_tensor *input, uint64_t offset,
 /* CommandBatch::matmul (ops.rs:242-373): out[m, n] = f16(sum_k input[m, k] *
  * weight[n, k]) with f32 accumulation (weight in the checkpoint's
  * [out_features, in_features] layout). Up to 32 rows run the library's
- * weight-streaming kernels; more rows run its tile GEMM as far as one output
- * tile per CU covers them, else (and for layouts those kernels do not read) a
+ * weight-streaming kernels; more rows run its tile GEMM where one output tile
+ * per CU covers them and measured faster, else (and for layouts those kernels
+ * do not read) a
  * hipBLASLt f16 GEMM with f32 compute, planned once per shape (or the few-row
  * kernel over groups of 8 rows when hipBLASLt has no solution for the shape). */
 mi_status mi_matmul(mi_batch *batch, const mi_tensor *input,

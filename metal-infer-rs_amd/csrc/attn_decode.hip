@@ -5,9 +5,10 @@
 // which grows with rows x keys, or would read K/V once per head chunk or token.
 //
 // Replaces the same reference kernels as the rows kernel (transformer.metal:
-// 1614-1665, 1824-2316) with the same precision: probabilities are f32 values
-// carried into the P V product as two f16 terms (hi + lo, 22 bits), partials and
-// their merge are f32.
+// 1614-1665, 1824-2316). Probabilities are f32 values carried into the P V product
+// as two f16 terms (hi + lo: 22 bits down to 2^-8 of the largest weight, 2^-31 of
+// it below, where the rows kernel multiplies the 24), partials and their merge are
+// f32; the error against 64 bits is the output's f16 rounding with both.
 //  - One workgroup per (key split, KV head and head chunk, sequence). Its
 //    waves take interleaved 32-key tiles, each with two register (K) and LDS
 //    (V) stages, the next tile in flight while one is computed.

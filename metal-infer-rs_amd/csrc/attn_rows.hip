@@ -18,8 +18,8 @@
 //    arrival counter: no cache-wide release fence, which on a multi-XCD part
 //    writes back the XCD's whole L2 and measured slower than a second
 //    launch), or attn_merge_kernel does in a second launch.
-// The batched decode at head_dim 128 has its own kernel further down
-// (attn_decode_stream_kernel: MFMA tiles, stream-K split).
+// The batched decode at head_dim 128, and at 64 where it measured faster, has its
+// own kernel further down (attn_decode_stream_kernel: MFMA tiles, stream-K split).
 #include <type_traits>
 
 #include "decode_tile.hpp"
@@ -658,12 +658,12 @@ typedef float sf4_t __attribute__((ext_vector_type(4)));
 // slower: 32 sequences of 1024 to 8192 keys 64.7 against 60.6 us).
 constexpr int kStreamPerCu = 2;
 
-// D = 64 keeps the precision of the rows kernel that served it: probabilities
-// are f32 values carried into P V as two f16 terms (hi + lo, 22 bits; twice the
-// P V MFMAs, which its bound, HBM, hides). Measured on MI355X, rows kernel ->
-// this with its merge launch: 70 sequences of 100 to 4000 keys, 32/8 heads 75.9
-// -> 71.1 us; 32 of 1024 to 8192 71.4 -> 60.6; 128 of 100 to 1500 66.8 -> 57.2;
-// 14 of 745 to 1456, 64/8 heads 31.6 -> 18.2.
+// At D = 64 probabilities are f32 values, as in the rows kernel that serves it too,
+// carried into P V as two f16 terms (hi + lo: 22 bits down to 2^-8 of the largest
+// weight, 2^-31 of it below; twice the P V MFMAs, which its bound, HBM, hides).
+// Measured on MI355X, rows kernel -> this with its merge launch: 64 sequences of 100
+// to 4000 keys, 40/8 heads 204 -> 66 us; 32 of them, 32/8 44 -> 36; 14 of 745 to
+// 1456, 64/8 31.6 -> 18.2.
 template <int D>
 __global__ __launch_bounds__(kStreamWaves * 64, kStreamPerCu) void attn_decode_stream_kernel(
     const RowsParams p) {

@@ -9,12 +9,13 @@
 // does, and walks 64-key K/V tiles staged into LDS by direct loads
 // (prefill_tile.hpp); the differences from that kernel keep the Tiled kind's
 // precision: probabilities are f32 values carried into P V as two f16 terms (hi +
-// lo, 22 bits; twice the P V MFMAs), and split partials are f32.
+// lo: 22 bits down to 2^-8 of the largest weight, 2^-31 of it below; twice the P V
+// MFMAs), and split partials are f32.
 //
 // A few tokens give one row tile per KV head, so the keys are split over the
-// chip and attn_tiled_merge_kernel, next on the stream, merges: with up to 32
-// partials of 128 rows an in-launch merge by the last arriver would read
-// megabytes through one CU.
+// chip and attn_tiled_merge_kernel, next on the stream, merges: with tens of
+// partials of 128 rows (one KV head: over a hundred) an in-launch merge by the last
+// arriver would read megabytes through one CU.
 #include <type_traits>
 
 #include "device_common.hpp"

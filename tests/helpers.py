@@ -6,7 +6,7 @@ import numpy as np
 import mi_attn
 import oracle
 
-# north_star: max-abs error <= 2e-3 against the reference CPU path (the f32
+# Max-abs error <= 2e-3 against the reference CPU path (the f32
 # oracle, unrounded), with f32 accumulation.
 TOL = 2e-3
 

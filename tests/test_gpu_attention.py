@@ -394,13 +394,20 @@ def stream_scratch_bytes(ctx, B, hq, hkv, limit=16 << 20):
     acc[128]) in each of 8 fixed slots per unit, one overflow slot per
     workgroup (2 per CU) and unit, and one u32 piece descriptor per unit; or,
     when that exceeds the buffer, the compact layout without the fixed
-    slots."""
+    slots. The group is cut into the fewest chunks of at most 16 heads, or,
+    where only their compact layout fits the buffer, the largest
+    power-of-two chunks that divide it."""
     g = hq // hkv
-    chunk = next(c for c in (16, 8, 4, 2, 1) if g % c == 0)
-    units = B * hkv * (g // chunk)
-    fixed = ((8 * units + 2 * ctx.compute_units + units) * chunk * 130 + units) * 4
-    compact = ((2 * ctx.compute_units + units) * chunk * 130 + units) * 4
-    return fixed if fixed <= limit else compact
+
+    def size(chunks, slots):
+        units, chunk = B * hkv * chunks, -(-g // chunks)
+        return (((slots + 1) * units + 2 * ctx.compute_units) * chunk * 130 + units) * 4
+
+    chunks = -(-g // 16)
+    dividing = next(c for c in range(chunks, g + 1) if g % c == 0 and (g // c) & (g // c - 1) == 0)
+    if size(chunks, 0) > limit >= size(dividing, 0):
+        chunks = dividing
+    return size(chunks, 8) if size(chunks, 8) <= limit else size(chunks, 0)
 
 
 def _batched_case(ctx, seed, B, hq, hkv, d, cap, lengths):
@@ -444,8 +451,8 @@ def test_batched_decode_gqa_ratios_and_ragged_lengths(ctx, hq, hkv, d):
 
 
 @pytest.mark.parametrize("B,hq,hkv,cap,lengths", [
-    # GQA 16 (one 16-head chunk), GQA 32 (two chunks), GQA 3 and 12 (chunks
-    # of 1 and 4), with zero-length sequences between others.
+    # GQA 16 (one 16-head chunk), GQA 32 (two chunks), GQA 3 and 12 (one
+    # chunk), with zero-length sequences between others.
     (6, 32, 2, 300, [300, 0, 17, 0, 299, 1]),
     (3, 64, 2, 520, [520, 7, 519]),
     (4, 12, 4, 260, [0, 260, 33, 129]),

@@ -14,10 +14,15 @@ def rand(seed, shape, scale=1.0):
     return (scale * np.random.default_rng(seed).standard_normal(shape)).astype(np.float16).view(np.uint16)
 
 
+# Splits and keys per split of the cases below that are there for them (256 CUs).
+SPLITS = {(64, 31): (1, 32), (64, 128): (2, 96), (64, 384): (4, 128), (64, 4999): (32, 160), (8, 9000): (71, 128)}
+
+
 @pytest.mark.parametrize("hq,hkv,d,T,off,extra,causal,kind", [
     (8, 1, 128, 1, 0, 0, True, "flash-decode"),        # one key
     (64, 8, 128, 1, 31, 0, True, "decode-split-kv"),   # one whole tile, one split
-    (64, 8, 128, 1, 128, 0, True, "flash-decode"),     # a second split of one key
+    (64, 8, 128, 1, 128, 0, True, "flash-decode"),     # 129 keys: splits of 96 and 33
+    (64, 8, 128, 1, 384, 0, True, "flash-decode"),     # a fourth split of one key
     (32, 8, 128, 1, 255, 9, True, "flash-decode"),     # keys past the window are not read
     (32, 8, 128, 1, 99, 57, False, "flash-decode"),    # non-causal: every key
     (64, 8, 128, 1, 4999, 0, True, "flash-decode"),    # 32 splits: a whole merge pass
@@ -38,6 +43,8 @@ def test_few_row_attention(ctx, hq, hkv, d, T, off, extra, causal, kind):
     geo = dict(hq=hq, hkv=hkv, d=d, off=off, causal=causal)
     qt, (ko, kview) = ctx.tensor(q), upload_kv(ctx, k, "head_major")
     info = ctx.plan(qt, kview, kview, mi_attn.AttentionConfig(hq, hkv, d, causal, off), KINDS[kind])
+    if (hq, off) in SPLITS:
+        assert (info["splits"], info["block_keys"]) == SPLITS[hq, off], info
     group, chunks = hq // hkv, 1 if T > 1 else -(-hq // hkv // 16)
     rows = T * -(-group // chunks)
     assert info["kernel"] == "attn_decode" and info["block_threads"] == 512 and info["grid"][1] == hkv * chunks, info

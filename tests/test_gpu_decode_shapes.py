@@ -1,9 +1,9 @@
 """Seeded random batched-decode geometries against the oracle: 1-48
-sequences, GQA ratios 1-16, head_dim 128 (the stream-K MFMA kernel and its
-merge launch) and 64 (the rows kernel), per-sequence lengths from 0 to past
-the cache capacity (clamped), head-major and token-major caches, the default
-plan and explicit split sizes (the rows kernel, splits merged inside the
-launch). Every sequence is checked (a zero-length one must be NaN, the
+sequences, GQA ratios 1-16, head_dim 128 (by default the stream-K MFMA kernel
+and its merge launch) and 64 (by default that or the rows kernel, by heads and
+units), per-sequence lengths from 0 to past the cache capacity (clamped),
+head-major and token-major caches, the default plan and explicit split sizes
+(the rows kernel, splits merged inside the launch). Every sequence is checked (a zero-length one must be NaN, the
 reference's 0/0), a second call must be bit-identical, and the
 no-allocation entry point must agree bit for bit where its buffer holds the
 partials."""
@@ -34,6 +34,29 @@ def _geometry(i: int):
     return rng, d, hkv * g, hkv, B, cap, lengths.astype(np.uint32), block, token_major
 
 
+# What each kind of call launches.
+KERNELS = {
+    "stream-128": ["attn_decode_stream", "attn_decode_stream_merge"],
+    "stream-64": ["attn_decode_stream", "attn_decode_stream_merge"],
+    "rows-default": ["attn_rows_batched"],
+    "rows-split": ["attn_rows_batched"],
+}
+
+
+def _kind(cus, i):
+    """The default at head_dim 64 is stream-K for groups of 8, for nine heads per CU, and for
+    groups of 4 whose rows splits come to six workgroups per CU, as long as there are at least
+    two KV heads, more keys than one rows split and no more units than stream workgroups."""
+    _, d, hq, hkv, B, cap, _, block, _ = _geometry(i)
+    if block != 0:
+        return "rows-split"
+    if d == 128:
+        return "stream-128"
+    g, units = hq // hkv, B * hkv
+    many = g == 8 or B * hq >= 9 * cus or (g == 4 and units * -(-cap // 768) >= 6 * cus)
+    return "stream-64" if cap > 768 and hkv > 1 and units <= 2 * cus and many else "rows-default"
+
+
 @pytest.mark.parametrize("i", range(CASES))
 def test_random_batched_decode_geometry(ctx, i):
     rng, d, hq, hkv, B, cap, lengths, block, token_major = _geometry(i)
@@ -53,11 +76,18 @@ def test_random_batched_decode_geometry(ctx, i):
     label = (f"case {i}: d={d} hq={hq} hkv={hkv} B={B} cap={cap} block={block} "
              f"token_major={token_major}")
     outs = []
-    for _ in range(2):
-        batch = ctx.begin_batch()
-        out = batch.attention_decode_batched(qt, kview, vview, lt, cfg, block)
-        batch.finish()
-        outs.append(ctx.download(out))
+    ctx.take_kernel_profiles()
+    ctx.set_kernel_profiling(True)
+    try:
+        for _ in range(2):
+            batch = ctx.begin_batch()
+            out = batch.attention_decode_batched(qt, kview, vview, lt, cfg, block)
+            batch.finish()
+            outs.append(ctx.download(out))
+        names = [name for name, _ in ctx.take_kernel_profiles()]
+    finally:
+        ctx.set_kernel_profiling(False)
+    assert names == KERNELS[_kind(ctx.compute_units, i)] * 2, (label, names)
     got = outs[0]
     assert np.array_equal(got.view(np.uint16), outs[1].view(np.uint16)), label
     for b in range(B):
@@ -79,17 +109,18 @@ def test_random_batched_decode_geometry(ctx, i):
         assert np.array_equal(ctx.download(fixed).view(np.uint16), got.view(np.uint16)), label
 
 
-def test_random_decode_geometries_cover_both_kernels():
-    """The sample above holds stream-K calls (head_dim 128, default plan),
-    rows-kernel calls by default (head_dim 64) and with explicit splits,
-    both cache layouts, zero lengths and lengths past the capacity."""
+def test_random_decode_geometries_cover_every_route():
+    """The sample above holds stream-K calls at both head dimensions, default
+    calls that stay on the rows kernel and explicit splits (each call is checked
+    to have run its kernels), both cache layouts, zero lengths and lengths past
+    the capacity."""
     kinds, layouts, zero, clamped = set(), set(), 0, 0
     for i in range(CASES):
-        _, d, _, _, _, cap, lengths, block, token_major = _geometry(i)
-        kinds.add("stream" if d == 128 and block == 0 else "rows-default" if block == 0 else "rows-split")
+        _, _, _, _, _, cap, lengths, _, token_major = _geometry(i)
+        kinds.add(_kind(256, i))
         layouts.add(token_major)
         zero += int((lengths == 0).any())
         clamped += int((lengths > cap).any())
-    assert kinds == {"stream", "rows-default", "rows-split"}, kinds
+    assert kinds == set(KERNELS), kinds
     assert layouts == {True, False}
     assert zero > 0 and clamped > 0
