@@ -288,9 +288,8 @@ mi_status mi_attention_plan(const mi_context *ctx, const mi_tensor *q,
  * block_keys = 0 picks the default: at head_dim 128 with B <= 1024 an MFMA
  * kernel whose workgroups share all sequences' keys equally (stream-K; few
  * keys: one piece of a unit per workgroup), and at 64 too where short
- * sequences would not make it the slower one (groups of 8, or many heads, and
- * at most 2 units per CU); otherwise the rows kernel over a flat (sequence,
- * KV head, split) grid.
+ * sequences would not make it the slower one (groups of 8, or many heads);
+ * otherwise the rows kernel over a flat (sequence, KV head, split) grid.
  * block_keys > 0 runs the rows kernel with splits of that many keys. */
 mi_status mi_attention_decode_batched(mi_batch *batch, const mi_tensor *q,
                                       const mi_tensor *k, const mi_tensor *v,

@@ -732,11 +732,17 @@ __global__ __launch_bounds__(kStreamWaves * 64, kStreamPerCu) void attn_decode_s
   // keys, 16/8 heads 21.7 -> 13.2 us; 16 of 100 to 900, 32/8 28.1 -> 18.8; 4 of
   // 3000 to 5000 30.8 -> 26.0; 128 of 10 to 100 77.9 -> 42.6; 512-key pieces lost
   // where they run (20 of 500 to 1500: 28.7 against 25.7 in segments).
+  // Where no sequence is longer than one piece, a workgroup takes several of them
+  // in turn if there are more than workgroups: equal segments of at least 128 keys
+  // would hold up to 128 units each (70 sequences of one key, 40/8 heads 400 -> 15.9
+  // us; 128 of 20 keys 37.4 -> 18.8).
   uint32_t piece_keys = 0;
-  if (s_pre[p.batch] <= (uint64_t)gridDim.x * kStreamPieceMost) {
+  if (s_pre[p.batch] <= max((uint64_t)gridDim.x * kStreamPieceMost, (uint64_t)p.batch * upb * kStreamMinKeys)) {
     uint32_t count[2] = {0, 0};  // pieces of kStreamMinKeys and of kStreamPieceMost keys
+    uint32_t used = 0;           // sequences with a key
     for (uint32_t c0 = 0; c0 < p.batch; c0 += 64) {
       const uint32_t n = c0 + lane < p.batch ? s_len[c0 + lane] : 0;
+      used += (uint32_t)__popcll(__ballot(n != 0));
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const uint32_t size = i == 0 ? kStreamMinKeys : kStreamPieceMost;
@@ -747,7 +753,7 @@ __global__ __launch_bounds__(kStreamWaves * 64, kStreamPerCu) void attn_decode_s
       }
     }
     if ((uint64_t)count[1] * upb <= gridDim.x) piece_keys = kStreamPieceMost;
-    if ((uint64_t)count[0] * upb <= gridDim.x) piece_keys = kStreamMinKeys;
+    if ((uint64_t)count[0] * upb <= gridDim.x || count[0] == used) piece_keys = kStreamMinKeys;
   }
   if (piece_keys != 0) {
     __syncthreads();
@@ -773,8 +779,8 @@ __global__ __launch_bounds__(kStreamWaves * 64, kStreamPerCu) void attn_decode_s
         p.out[(int64_t)b * p.o_seq + (int64_t)(idx / D) * p.o_head + idx % D] = 0x7e00;
   const uint64_t total = s_pre[p.batch];
   // At least kStreamMinKeys per workgroup; the rest of the grid idles.
-  // (Pieces: one position per workgroup.)
-  const uint64_t W = piece_keys != 0 ? max((uint64_t)1, total) : min((uint64_t)gridDim.x, max((uint64_t)1, total / kStreamMinKeys));
+  // (Pieces: one position per workgroup, or whole units.)
+  const uint64_t W = min((uint64_t)gridDim.x, max((uint64_t)1, piece_keys != 0 ? total : total / kStreamMinKeys));
   // 32-bit division when the total fits (a 64-bit one is a long sequence).
   const uint64_t seg = total + W - 1 <= 0xffffffffull
                            ? (uint64_t)((uint32_t)(total + W - 1) / (uint32_t)W)

@@ -44,17 +44,19 @@ KERNELS = {
 
 
 def _kind(cus, i):
-    """The default at head_dim 64 is stream-K for groups of 8, for nine heads per CU, and for
-    groups of 4 whose rows splits come to six workgroups per CU, as long as there are at least
-    two KV heads, more keys than one rows split and no more units than stream workgroups."""
+    """The default at head_dim 64 is stream-K for groups of 8, for larger groups than 4 of nine
+    heads per CU, and for groups of 4 whose rows splits come to six workgroups per CU (not
+    between one unit and six per CU), as long as there are at least
+    two KV heads and more keys than one rows split."""
     _, d, hq, hkv, B, cap, _, block, _ = _geometry(i)
     if block != 0:
         return "rows-split"
     if d == 128:
         return "stream-128"
     g, units = hq // hkv, B * hkv
-    many = g == 8 or B * hq >= 9 * cus or (g == 4 and units * -(-cap // 768) >= 6 * cus)
-    return "stream-64" if cap > 768 and hkv > 1 and units <= 2 * cus and many else "rows-default"
+    four = g == 4 and units * -(-cap // 768) >= 6 * cus and not cus < units < 6 * cus
+    many = g == 8 or (g > 4 and B * hq >= 9 * cus) or four
+    return "stream-64" if cap > 768 and hkv > 1 and many else "rows-default"
 
 
 @pytest.mark.parametrize("i", range(CASES))

@@ -50,6 +50,10 @@ def run(ctx, q, k, v, lengths, hq, hkv, d, cap):
     (40, 8, 64, 800, [(b * 97) % 250 for b in range(60)] + [800]),  # groups of 5, pieces
     (34, 2, 64, 800, [(b * 97) % 801 for b in range(70)]),          # chunks of 9 and 8
     (8, 2, 64, 8192, [(b * 97) % 300 for b in range(90)]),          # groups of 4 by the capacity
+    (64, 8, 64, 800, [(b * 5) % 129 for b in range(150)]),          # whole units, several per workgroup
+    (16, 8, 128, 130, [(b * 5) % 129 for b in range(150)]),
+    (16, 8, 128, 130, [(b * 5) % 130 for b in range(150)]),         # one key too many: equal segments
+    (8, 4, 128, 20, [1] * 600),
 ])
 def test_batched_decode_work_split(ctx, hq, hkv, d, cap, lengths):
     B = len(lengths)
@@ -87,8 +91,7 @@ def test_batched_decode_of_wide_groups_in_the_fixed_buffer(ctx, B, hq, hkv, cap)
 @pytest.mark.parametrize("hq,hkv,cap,B", [
     (32, 8, 4096, 8),    # groups of 4, few sequences
     (32, 8, 1024, 32),   # two rows splits of each unit
-    (32, 8, 1024, 70),   # more units than workgroups
-    (64, 8, 1024, 70),
+    (32, 8, 4096, 70),   # groups of 4, between one unit and six per CU
     (40, 8, 1024, 8),    # fewer than nine heads per CU
     (16, 8, 1024, 20),
     (8, 1, 4096, 8),     # one KV head
