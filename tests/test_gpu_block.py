@@ -451,7 +451,8 @@ def test_rope_aligned_and_unaligned_rows_agree_bit_for_bit(ctx):
     # The same rows 8 bytes past a 16-byte boundary: a view at offset 4 halves.
     store = np.zeros(T * H * D + 8, dtype=np.uint16)
     store[4:4 + T * H * D] = x.reshape(-1)
-    shifted = ctx.tensor(store).view((T, H, D), (H * D, D, 1), offset=4)
+    dev = ctx.tensor(store)  # the view does not own the memory
+    shifted = dev.view((T, H, D), (H * D, D, 1), offset=4)
     unaligned = ctx.download(ctx.rope(shifted, 40, 1e6))
     assert (aligned == unaligned).all()
     assert (np.abs(f16(aligned).astype(np.float64) - f16(oracle.rope(x, offset=40, theta=1e6)))
