@@ -798,38 +798,48 @@ mi_status decode_batched(mi_batch *batch, const mi_tensor *q, const mi_tensor *k
   // device data, and the capacity says nothing of them, so the line is drawn by
   // what the host knows. The rows kernel spends vector arithmetic by heads and
   // reads K/V again for each of its head chunks; the stream kernel has the longer
-  // fixed chain and a second launch. Measured on MI355X over lengths from 1 to 8192 in capacities of 1024 to
-  // 8192 (rows / stream us): groups of 8, 8 sequences of 64/8 heads, 1 key 8.1 /
-  // 8.9, 20 keys 8.8 / 9.0, 700 keys 20.7 / 12.1; other groups from 9 heads per CU on, 64 sequences of
-  // 40/8 heads, 20 keys 23.4 / 9.8, 100 to 4000 keys 204 / 66; groups of 4 where the
-  // rows kernel's empty splits come to 6 workgroups per CU, 32 sequences of 32/8 heads
-  // in 4096, 20 keys 9.1 / 8.4, 100 to 4000 keys 44 / 36, but in 1024, 20 keys 7.2 /
-  // 8.5, and not between one unit and 6 per CU (64 of them in 8192, 40 to 1000 keys
-  // 29.8 / 34.8). Not: 8 sequences of 40/8 heads, 20 keys
-  // 5.5 / 8.6; 32 of 16/8 5.3 / 8.1, 200 of 16/8 14.5 / 18.9. In a capacity of one
-  // rows split nothing is merged (one sequence of 60 keys 4.4 / 8.0).
+  // fixed chain and a second launch. Measured on MI355X over lengths from 1 to 8192
+  // in capacities of 1024 to 8192 (rows / stream us): groups of 8, 8 sequences of
+  // 64/8 heads, 1 key 8.1 / 8.9, 20 keys 8.8 / 9.0, 700 keys 20.7 / 12.1; other groups
+  // from 9 heads per CU on, 64 sequences of 40/8 heads, 20 keys 23.4 / 9.8, 100 to
+  // 4000 keys 204 / 66; groups of 4 where the rows kernel's empty splits come to 6
+  // workgroups per CU, 32 sequences of 32/8 heads in 4096, 20 keys 9.1 / 8.4, 100 to
+  // 4000 keys 44 / 36, but in 1024, 20 keys 7.2 / 8.5, and not between one unit and 6
+  // per CU (64 of them in 8192, 40 to 1000 keys 29.8 / 34.8). Not: 8 sequences of
+  // 40/8 heads, 20 keys 5.5 / 8.6; 32 of 16/8 5.3 / 8.1, 200 of 16/8 14.5 / 18.9. In a
+  // capacity of one rows split nothing is merged (one sequence of 60 keys 4.4 / 8.0).
+  // Past the no-allocation buffer, which the rows kernel's partials fill by the
+  // capacity and the stream kernel's by the heads alone, both entry points take the
+  // kernel whose partials fit it (in 8192, 250 sequences of 32/8 heads, 20 keys 33.1 /
+  // 23.0, 4000 keys 372 / 317; 500 of 16/8, 20 keys 43.9 / 36.3, 4000 keys 653 / 621,
+  // though 40 to 1000 keys 94 / 123).
   const uint64_t cus = std::max<uint32_t>(batch->ctx->compute_units, 1);
   const uint64_t kv_units = (uint64_t)B * p.Hkv;
+  const uint64_t rows_splits = ceil_div(p.L, kRowsBatchedBlock);
+  rp.group = p.G, rp.stream_workgroups = kernels::stream_workgroups(batch->ctx->compute_units);
+  auto partial_bytes = [&](uint32_t chunks, uint32_t slots) -> uint64_t {
+    return kernels::stream_partial_floats(kv_units * chunks, rp.stream_workgroups, ceil_div(p.G, chunks),
+                                          slots, p.D) *
+           sizeof(float);
+  };
+  const uint32_t fewest_chunks = std::max(1u, ceil_div(p.G, kernels::kDecodeRows));
   const bool stream64 =
-      p.D == 64 && p.L > kRowsBatchedBlock && p.Hkv > 1 &&
-      (p.G == 8 || (p.G > 4 && kv_units * p.G >= 9 * cus) ||
-       (p.G == 4 && kv_units * ceil_div(p.L, kRowsBatchedBlock) >= 6 * cus &&
-        (kv_units <= cus || kv_units >= 6 * cus)));
+      p.D == 64 && rows_splits > 1 &&
+      ((p.Hkv > 1 && (p.G == 8 || (p.G > 4 && kv_units * p.G >= 9 * cus) ||
+                      (p.G == 4 && kv_units * rows_splits >= 6 * cus &&
+                       (kv_units <= cus || kv_units >= 6 * cus)))) ||
+       ((p.G >= 4 || kv_units >= 128) &&
+        kv_units * p.G * rows_splits * (p.D + 2) * sizeof(float) > kNoAllocScratchBytes &&
+        partial_bytes(fewest_chunks, 0) <= kNoAllocScratchBytes));
   const bool stream = block_keys == 0 && (uint64_t)B <= kernels::kStreamMaxBatch &&
                       pos_stride_fits_u32(k->stride[1], v->stride[1], 32) && (p.D == 128 || stream64);
   if (stream) {
-    rp.group = p.G, rp.stream_workgroups = kernels::stream_workgroups(batch->ctx->compute_units);
-    auto partial_bytes = [&](uint32_t chunks, uint32_t slots) -> uint64_t {
-      return kernels::stream_partial_floats(kv_units * chunks, rp.stream_workgroups, ceil_div(p.G, chunks),
-                                            slots, p.D) *
-             sizeof(float);
-    };
     // The fewest head chunks, each of which reads K/V: unless their partials pass
     // the no-allocation buffer where those of the largest power-of-two chunks that
     // divide the group fit it (more chunks, but smaller overflow slots). The choice
     // moves the pieces' boundaries and so the rounding, and is the same with and
     // without that buffer.
-    rp.head_chunks = std::max(1u, ceil_div(p.G, kernels::kDecodeRows));
+    rp.head_chunks = fewest_chunks;
     if (partial_bytes(rp.head_chunks, 0) > kNoAllocScratchBytes) {
       uint32_t chunks = rp.head_chunks;
       while (p.G % chunks != 0 || !pow2(p.G / chunks)) ++chunks;

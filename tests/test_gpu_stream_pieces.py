@@ -88,6 +88,45 @@ def test_batched_decode_of_wide_groups_in_the_fixed_buffer(ctx, B, hq, hkv, cap)
         assert_parity(got[b:b + 1], ref, label=f"seq {b} len {n}")
 
 
+@pytest.mark.parametrize("B,hq,hkv,cap,fits", [
+    (190, 32, 8, 8192, False),  # groups of 4, whose units alone keep to the rows kernel
+    (190, 32, 8, 7680, True),   # one rows split fewer
+    (500, 16, 8, 8192, False),  # groups of 2
+    (1000, 8, 8, 6200, False),  # groups of 1
+    (1000, 8, 1, 6200, False),  # one KV head
+])
+def test_calls_past_the_fixed_buffer_by_their_capacity_take_the_kernel_that_fits(ctx, B, hq, hkv, cap, fits):
+    """The rows kernel's partials grow with the capacity; where they pass the no-allocation buffer the
+    stream kernel serves both calls. All sequences read one cache."""
+    d, lengths = 64, [1 + (7 * b) % 900 for b in range(B)]
+    assert (B * hq * -(-cap // 768) * (d + 2) * 4 <= 16 << 20) == fits
+    q, k, v = rand(1, (B, hq, d), 2.0), rand(2, (cap, hkv, d)), rand(3, (cap, hkv, d))
+    qt, lt = ctx.tensor(q), ctx.tensor(np.asarray(lengths, np.uint32), mi_attn.U32)
+    ks, vs = ctx.tensor(k), ctx.tensor(v)  # the views do not own the memory
+    kt, vt = (x.view((B, cap, hkv, d), (0, hkv * d, d, 1)) for x in (ks, vs))
+    cfg = mi_attn.AttentionConfig(hq, hkv, d, True, 0)
+    ctx.take_kernel_profiles()
+    ctx.set_kernel_profiling(True)
+    try:
+        batch = ctx.begin_batch()
+        out = batch.attention_decode_batched(qt, kt, vt, lt, cfg)
+        batch.finish()
+        names = [name for name, _ in ctx.take_kernel_profiles()]
+    finally:
+        ctx.set_kernel_profiling(False)
+    assert names == (["attn_rows_batched"] if fits else ["attn_decode_stream", "attn_decode_stream_merge"]), names
+    fixed = ctx.empty(q.shape)
+    batch = ctx.begin_batch()
+    batch.attention_decode_batched_noalloc(qt, kt, vt, lt, cfg, 0, fixed)
+    batch.finish()
+    got = ctx.download(out)
+    assert (ctx.download(fixed) == got).all()
+    for b in range(0, B, 97):
+        n = lengths[b]
+        ref = oracle_attention(q[b:b + 1], k[:n], v[:n], hq=hq, hkv=hkv, d=d, off=n - 1)
+        assert_parity(got[b:b + 1], ref, label=f"seq {b} len {n}")
+
+
 @pytest.mark.parametrize("hq,hkv,cap,B", [
     (32, 8, 4096, 8),    # groups of 4, few sequences
     (32, 8, 1024, 32),   # two rows splits of each unit
