@@ -423,8 +423,7 @@ mi_status mi_rope(mi_batch *batch, const mi_tensor *input, uint64_t offset,
  * [out_features, in_features] layout). Up to 32 rows run the library's
  * weight-streaming kernels; more rows run its tile GEMM where one output tile
  * per CU covers them and measured faster, else (and for layouts those kernels
- * do not read) a
- * hipBLASLt f16 GEMM with f32 compute, planned once per shape (or the few-row
+ * do not read) a hipBLASLt f16 GEMM with f32 compute, planned once per shape (or the few-row
  * kernel over groups of 8 rows when hipBLASLt has no solution for the shape). */
 mi_status mi_matmul(mi_batch *batch, const mi_tensor *input,
                     const mi_tensor *weight, const mi_tensor *out);
